@@ -188,9 +188,9 @@ def traffic_from_profile(name: str):
         return None
 
 
-# The kernel matmul_backward launches for aligned shapes with a 256 x 128 tile
-# per CU (2048^3 and the non-square C2 case): dA and dB tiles in one grid.
-HEAD_KERNEL = "matmul_backward_stream"
+# The kernel matmul_backward launches for products above 2^24 multiply-adds:
+# dA and dB tiles in one grid.
+HEAD_KERNEL = "gemm_pair_kernel"
 COPY_PROBE_BYTES = 256 << 20  # calibration copy: reads and writes this many bytes
 
 
@@ -420,11 +420,11 @@ def trace_summary(trace_csv: str, bench_out: str) -> str:
     with open(trace_csv) as f:
         rows = sorted(csv.DictReader(f), key=lambda r: int(r["Start_Timestamp"]))
 
-    def seq(part, grid=None):
+    def seq(part):
         return [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in rows
-                if part in r["Kernel_Name"] and (grid is None or int(r["Grid_Size_X"]) == grid)]
+                if part in r["Kernel_Name"]]
 
-    c2, c2p = seq(HEAD_KERNEL, 256 * 512), seq(HEAD_KERNEL, 512 * 512)
+    c2 = seq(HEAD_KERNEL)
     relu, fin, adam = seq("colreduce_pass1<true"), seq("colreduce_finalize"), seq("adam_kernel")
     # 2048^3 dispatches in launch order: per region its untimed launches, 4
     # queue-ahead, K timed; the same for the resident region; one check
@@ -434,6 +434,7 @@ def trace_summary(trace_csv: str, bench_out: str) -> str:
     t0 = a + 4
     r0 = t0 + K + b + 4
     c, _ = warm["C2'"]
+    c2p = c2[r0 + K + 1 + 4:]  # the check launch, then C2' (whose grid is the same) with 4 ahead
     e, _ = warm["C3 relu"]
     g, _ = warm["C3 Adam"]
     both = [x + y for x, y in zip(relu[e:e + K], fin[e:e + K])]
@@ -1214,7 +1215,7 @@ def bench_rows(ctx, rng, steps: int, warmup: int, cpu: bool = True) -> list:
     k = n_sets(4.0 * (T_ * In + Out * In + 2 * T_ * Out))
     xw_, W_, bb_ = Rot(ctx, k, xw), Rot(ctx, k, W), Rot(ctx, k, bb)
     yw_ = Rot(ctx, k, shape=(T_, Out))
-    record("a26", "Linear::forward (fused)", "gemm_stream_kernel (bias epilogue)",
+    record("a26", "Linear::forward (fused)", "gemm_kernel (bias epilogue)",
            "[4096,512]x[512,2048]",
            flops=2.0 * T_ * In * Out,
            launch=lambda i: ctx._check(L.load().numrs_hip_linear_forward(
@@ -1227,7 +1228,7 @@ def bench_rows(ctx, rng, steps: int, warmup: int, cpu: bool = True) -> list:
     gw_, dxw_ = Rot(ctx, k, gw), Rot(ctx, k, shape=(T_, In))
     dW_, db_ = Rot(ctx, k, shape=(Out, In)), Rot(ctx, k, shape=(Out,))
     record("a10+a11+a5", "Linear backward (fused)",
-           "linear_backward_stream_small (split reduction and bias sums in the launch)",
+           "gemm_pair_kernel + splitk_reduce (bias sums in the same launch)",
            "[4096,512]x[512,2048]", flops=4.0 * T_ * In * Out,
            launch=lambda i: ctx._check(L.load().numrs_hip_linear_backward(
                ctx.handle, gw_[i].ptr, xw_[i].ptr, W_[i].ptr, dxw_[i].ptr, dW_[i].ptr, db_[i].ptr,
@@ -1301,7 +1302,7 @@ def bench_rows(ctx, rng, steps: int, warmup: int, cpu: bool = True) -> list:
            note="one persistent launch for all 128 steps of both layers, the first layer's "
                 "input projection inside the steps; no numrs CPU path")
     record("N4", "LSTM x2 backward (new op)",
-           "lstm2_bwd_prep + lstm2_bwd_persist + 2 x (tn_pair_stream_small + splitk_reduce)",
+           "lstm2_bwd_prep + lstm2_bwd_persist + 2 x (gemm_pair_kernel + splitk_reduce)",
            f"B {B5}, T {T5}, in {I5}, hidden {H5} (C5)", flops=bwd_flops, launch=lstm_bwd,
            note="one persistent launch for all 128 steps of both layers (bias partials formed "
                 "in the steps), then each layer's dW_ih and dW_hh over all steps as one paired "

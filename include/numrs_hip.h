@@ -220,12 +220,12 @@ int numrs_hip_matmul(numrs_hip_ctx *ctx, const float *A, const float *B, float *
 
 /* No counterpart in the reference: where the products of one call cut their
  * reduction into split-K ranges (weight gradients over many tokens), how the
- * partial products are added.  FUSED (the default): inside the products' own
- * launch -- the grid's last workgroups (or the last split to arrive) add each
- * output block's partials once all of its splits have stored them, with no
- * workgroup waiting for another.  SEPARATE: one more launch after the
- * products.  Both add the splits in the same order with the same
- * arithmetic: the same bits. */
+ * partial products of small products (at most 2^24 multiply-adds) are added.
+ * FUSED (the default): inside the products' own launch -- the last split of
+ * an output block to arrive adds the block's partials, with no workgroup
+ * waiting for another.  SEPARATE: one more launch after the products, as
+ * larger products take in both modes.  Both add the splits in the same order
+ * with the same arithmetic: the same bits. */
 #define NUMRS_HIP_SPLIT_REDUCE_FUSED 0
 #define NUMRS_HIP_SPLIT_REDUCE_SEPARATE 1
 int numrs_hip_set_split_reduction(numrs_hip_ctx *ctx, int mode);

@@ -249,7 +249,7 @@ struct BatchedOut {
 };
 
 // C1_z = alpha X_z Y1_z ([M,K] x [K,N]) and C2_z = alpha X_z^T Y2_z
-// ([K,M] x [M,N]) for z < batch, in one launch where the streamed path fits
+// ([K,M] x [M,N]) for z < batch, in one launch
 // (the shape of the Linear backward and of attention's dQ/dK).  Either
 // output may be null; accumulate adds into the outputs.
 int gemm_nn_tn_pair(numrs_hip_ctx *ctx, BatchedMat X, BatchedMat Y1, BatchedOut C1, BatchedMat Y2,
@@ -268,7 +268,7 @@ int cross_entropy_loss_impl(numrs_hip_ctx *ctx, const float *logits, const float
 bool cross_entropy_preforms(int64_t B);
 
 // C1_z = alpha1 X1_z^T Y1_z and C2_z = alpha2 X2_z^T Y2_z (X [M,K], Y [M,N],
-// C [K,N]) for z < batch, in one launch where the streamed path fits
+// C [K,N]) for z < batch, in one launch
 // (attention's dV = P^T dO with dK = alpha dS^T Q).  Either output may be
 // null; accumulate adds into the outputs.
 int gemm_tn_pair(numrs_hip_ctx *ctx, BatchedMat X1, BatchedMat Y1, BatchedOut C1, float alpha1,
@@ -276,7 +276,7 @@ int gemm_tn_pair(numrs_hip_ctx *ctx, BatchedMat X1, BatchedMat Y1, BatchedOut C1
                  int64_t N, int accumulate, int64_t batch, int64_t binner);
 // Two weight gradients of one left operand, C1[K,N1] = X^T Y1 and
 // C2[K,N2] = X^T Y2 (X [M,K] at row stride ldx, Y1 [M,N1], Y2 [M,N2]), in
-// one launch with a joint split plan where the streamed path fits, and the
+// one launch with a joint split plan, and the
 // column sums db[K] of X (null for none) formed by the launch that reduces
 // the splits (the LSTM's dW_ih, dW_hh and db): from db_part [db_rows, K],
 // partial sums of X over row groups added in row order as a compensated sum,

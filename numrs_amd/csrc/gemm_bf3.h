@@ -1,0 +1,380 @@
+// Products of fp32 matrices on the bf16 matrix cores, at fp32 accuracy.
+//
+// An fp32 value is the sum of three bf16 values, x = h + m + l with h = bf16(x),
+// m = bf16(x - h), l = x - h - m (round to nearest even; both differences are exact, and
+// what is left after two roundings fits bf16's 8 bits).  A product is then
+//   x y = hx hy + (hx my + mx hy) + (mx my + hx ly + lx hy) + [mx ly + lx my + lx ly],
+// the bracket, at most 2^-26 |x y|, left out: six v_mfma_f32_16x16x32_bf16 per 16 x 16 x 32
+// block, accumulated in fp32, smallest terms first, from zero for every 32 reduction steps;
+// the sums of 32 steps are added into fp32 totals.  Measured against float64 on N(0, 1)
+// operands, relative 2-norm error at R = 256 | 512 | 2048 reduction steps: 0.7 | 0.9 |
+// 1.5e-7, where v_mfma_f32_32x32x2f32 with totals every 96 steps has 1.9 | 1.9 | 2.0e-7.
+//
+// What bounds it: gfx950's bf16 MFMA rate is 2.5 PFLOP/s against 157 TFLOP/s for fp32
+// MFMAs, so six of them take 0.38 of the time at nominal rates.  On N(0, 1) data the card
+// lowers its clock under them (about 2.0 GHz; the same launches on zeros run 1.36 times as
+// fast), and [4096, 2048] x [2048, 4096] runs at 176-184 TFLOP/s of fp32 work = 1.1 PFLOP/s
+// of bf16 (hipBLASLt's plain bf16 product of that size: 1.14; the fp32 MFMA kernel that
+// this replaced: 142 TFLOP/s).
+//
+// Special values.  An infinity, a NaN or a magnitude above bf16's largest finite value has
+// a term x - h that is not finite, and makes every output of its row or column NaN or
+// infinite.  A wave that finds such an output recomputes its block with fp32 MFMAs, so
+// that the results are those of fp32 arithmetic.  Below 2^-110 the terms m and l lose bits
+// to bf16's smallest subnormal, 2^-133: an absolute error of at most 2^-134 per operand.
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+
+namespace bf3 {
+
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+// at any float's address: rows of odd length need no path of their own
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+// (a, b) -> the three terms of each, packed in pairs.
+__device__ __forceinline__ void split2(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+  auto pack = [](float x, float y) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, b2));
+  };
+  auto lo = [](uint32_t v) { return __builtin_bit_cast(float, v << 16); };
+  auto hi = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); };
+  h = pack(a, b);
+  const float ra = a - lo(h), rb = b - hi(h);
+  m = pack(ra, rb);
+  l = pack(ra - lo(m), rb - hi(m));
+}
+
+constexpr int kBR = 32;           // reduction steps per tile (one MFMA's)
+constexpr int kChunks = kBR / 8;  // 16-byte chunks (8 bf16) of a row
+
+// LDS image of an EXT x kBR operand tile: three planes (h, m, l) of [chunk][row] 16-byte
+// chunks.  Row r of chunk ch sits at slot r ^ swizzle(ch): the 16 rows x 4 chunks of one
+// MFMA operand read fall on different banks, and so do the 4 chunks x 4 rows that 16 lanes
+// write when their rows are contiguous in memory.
+template <int EXT>
+struct Tile {
+  static constexpr int kChunkStride = EXT * 16;
+  static constexpr int kPlane = kChunks * kChunkStride;
+  static constexpr int kBytes = 3 * kPlane;
+};
+__device__ __forceinline__ int swizzle(int ch) { return ((ch & 1) ? 12 : 0) ^ ((ch & 2) ? 4 : 0); }
+
+// A thread's share of an EXT x kBR tile of an operand that is reduction-contiguous (RC:
+// base[row ld + r]) or not (base[r ld + row]): N units of 8 consecutive reduction steps of
+// one row.  Rows past the operand's last one read the last one (their products are not
+// stored).  WIDE: 64-bit offsets, for leading dimensions of 2^24 and more.
+template <bool RC, int EXT, int NT, bool WIDE>
+struct Loader {
+  static constexpr int N = EXT * kChunks / NT;
+  static_assert(N >= 1 && N * NT == EXT * kChunks, "whole units");
+  static constexpr bool kPairs = !RC && N == 2;  // two units: neighbouring rows, loaded together
+  static_assert(RC || kPairs || EXT % 64 == 0, "one chunk per wave");
+  using Off = typename std::conditional<WIDE, int64_t, uint32_t>::type;
+  float v[N][8];
+  Off off[N];   // element offset of the unit's row (and, RC, its chunk) from the tile base
+  int slot[N];  // its byte offset in each plane of the LDS image
+
+  static __device__ __forceinline__ int row(int tid, int i) {
+    if (kPairs) return 2 * (tid % (EXT / 2)) + i;
+    const int u = tid + NT * i;
+    return RC ? u / kChunks : u % EXT;
+  }
+  static __device__ __forceinline__ int chunk(int tid, int i) {
+    if (kPairs) return tid / (EXT / 2);
+    const int u = tid + NT * i;
+    return RC ? u % kChunks : u / EXT;
+  }
+  // rows: how many of the tile's rows exist; at least 1, pairs: 2 (pairs_fit).  A pair whose
+  // first row is an odd last one reads the row before and that one, and trades places.
+  __device__ __forceinline__ void init(int tid, int64_t ld, int rows) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      int r = row(tid, i);
+      const int ch = chunk(tid, i);
+      const int put = kPairs && r - i > rows - 2 ? r ^ 1 : r;
+      slot[i] = ch * Tile<EXT>::kChunkStride + (put ^ swizzle(ch)) * 16;
+      r = kPairs ? min(r - i, rows - 2) + i : min(r, rows - 1);
+      off[i] = RC ? (Off)((Off)r * (Off)ld + (Off)(8 * ch)) : (Off)r;
+    }
+  }
+  // Unit i (pairs: both at i = 0) of the whole tile at `base`, row 0 of the tile at its first
+  // reduction step.
+  __device__ __forceinline__ void load(const float *base, int64_t ld, int tid, int i) {
+    if constexpr (RC) {
+      const f4u a = *reinterpret_cast<const f4u *>(base + off[i]);
+      const f4u b = *reinterpret_cast<const f4u *>(base + off[i] + 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[i][j] = a[j], v[i][4 + j] = b[j];
+    } else {
+      const int c = __builtin_amdgcn_readfirstlane(8 * chunk(tid, i));  // one chunk per wave
+      if constexpr (kPairs) {
+        if (i != 0) return;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const f2u a = *reinterpret_cast<const f2u *>((base + (c + j) * ld) + off[0]);
+          v[0][j] = a[0], v[1][j] = a[1];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[i][j] = (base + (c + j) * ld)[off[i]];
+      }
+    }
+  }
+  // The same for a tile of `left` <= kBR reduction steps; the others read as zero.
+  __device__ __forceinline__ void load_part(const float *base, int64_t ld, int tid, int i,
+                                            int left) {
+    const int c = 8 * chunk(tid, i);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const bool in = c + j < left;
+      const int64_t o = RC ? (int64_t)off[i] + (in ? j : -c) : (in ? (c + j) * ld : 0) + (int64_t)off[i];
+      const float x = base[o];
+      v[i][j] = in ? x : 0.0f;
+    }
+  }
+  // sign: 0, or the sign bit for the terms of -x (SIGNED).
+  template <bool SIGNED>
+  __device__ __forceinline__ void store(char *lds, int i, uint32_t sign) const {
+    auto at = [&](int j) {
+      return SIGNED ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i][j]) ^ sign) : v[i][j];
+    };
+    u4 h, m, l;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t a, b, c;
+      split2(at(2 * j), at(2 * j + 1), a, b, c);
+      h[j] = a, m[j] = b, l[j] = c;
+    }
+    char *p = lds + slot[i];
+    *reinterpret_cast<u4 *>(p) = h;
+    *reinterpret_cast<u4 *>(p + Tile<EXT>::kPlane) = m;
+    *reinterpret_cast<u4 *>(p + 2 * Tile<EXT>::kPlane) = l;
+  }
+};
+
+// One workgroup's output tile: WP x WQ waves of (16 BI) x (16 BJ) outputs.  Lane 16 g + c of
+// a wave holds, in tot[i][j][e], row 16 i + 4 g + e and column 16 j + c of the wave's block.
+template <int BI_, int BJ_, int WP_, int WQ_, bool WIDE_>
+struct Shape {
+  static constexpr int BI = BI_, BJ = BJ_, WP = WP_, WQ = WQ_;
+  static constexpr bool WIDE = WIDE_;
+  static constexpr int TP = 16 * BI * WP, TQ = 16 * BJ * WQ, NT = 64 * WP * WQ;
+  static constexpr int kStage = Tile<TP>::kBytes + Tile<TQ>::kBytes;
+  static constexpr int kLds = 2 * kStage;
+  // Whether an operand's last tile of TP (TQ) rows has enough of them for its loader.
+  static bool pairs_fit(bool rc, int64_t rows, int ext) {
+    return rc || ext * kChunks / NT != 2 || rows % ext != 1;
+  }
+};
+
+template <bool XRC, bool YRC, class S>
+struct Product {
+  static constexpr int BI = S::BI, BJ = S::BJ, TP = S::TP, TQ = S::TQ, NT = S::NT;
+  static_assert(BI % 2 == 0 && BJ % 2 == 0, "block pairs");
+  f4 tot[BI][BJ];
+
+  // tot = X Y over R >= 1 reduction steps; X: row 0 of the tile at the first step, rows_x of
+  // its TP rows exist (Y alike).  lds: S::kLds bytes.
+  //
+  // The MFMA's own sum rounds down rather than to nearest: its mean error is -6e-9 of the
+  // result's rms whatever the sign, which sums over many outputs (a bias gradient, a
+  // LayerNorm's statistics) would show (measured: 4 times the error of fp32 MFMAs in an
+  // encoder block's bias gradients).  So every other tile is formed from -Y and subtracted,
+  // and tiles whose `phase` differs in its last bit begin with the other sign: the mean error
+  // over 64 steps is 1e-10.
+  //
+  // A step of the loop multiplies one LDS stage while the next one is written.  Global loads
+  // run one step ahead in registers; each phase (one row block against all column blocks)
+  // splits and stores one unit and issues its next load.  The one barrier stands before the
+  // last phase: by then every wave has stored its share of the next stage and read its last
+  // row block of this one, so the last phase's MFMAs cover the first reads of the next stage.
+  __device__ __forceinline__ void run(const float *X, int64_t ldx, int rows_x, const float *Y,
+                                      int64_t ldy, int rows_y, int R, int phase, char *lds) {
+    using LX = Loader<XRC, TP, NT, S::WIDE>;
+    using LY = Loader<YRC, TQ, NT, S::WIDE>;
+    constexpr int kX = LX::N, kUnits = LX::N + LY::N;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 15, g = lane >> 4;
+    const int at = (c ^ swizzle(g)) * 16;
+    const int ax = g * Tile<TP>::kChunkStride + (wave / S::WQ) * (256 * BI) + at;
+    const int by = Tile<TP>::kBytes + g * Tile<TQ>::kChunkStride + (wave % S::WQ) * (256 * BJ) + at;
+    LX x;
+    LY y;
+    x.init(tid, ldx, rows_x);
+    y.init(tid, ldy, rows_y);
+    // A partial tile comes first, so that every later one is whole.
+    const int nk = (R + kBR - 1) / kBR, first = R - kBR * (nk - 1);
+    const int64_t xstep = XRC ? 1 : ldx, ystep = YRC ? 1 : ldy;
+    auto load = [&](int u, int kt) {  // kt >= 1
+      const int64_t r = first + (kt - 1) * (int64_t)kBR;
+      if (u < kX)
+        x.load(X + r * xstep, ldx, tid, u);
+      else
+        y.load(Y + r * ystep, ldy, tid, u - kX);
+    };
+    // Unit u of tile kt, whose Y is negated when kt + phase is odd.
+    auto store = [&](int u, int kt, char *s) {
+      if (u < kX)
+        x.template store<false>(s, u, 0);
+      else
+        y.template store<true>(s + Tile<TP>::kBytes, u - kX, (uint32_t)(kt + phase) << 31);
+    };
+    // Unit u's registers are free for its next load once the units it loads with are stored.
+    auto load_after = [&](int u, int kt) {
+      if (LX::kPairs && u < kX) {
+        if (u == kX - 1) load(0, kt);
+      } else if (LY::kPairs && u >= kX) {
+        if (u == kUnits - 1) load(kX, kt);
+      } else {
+        load(u, kt);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) tot[i][j] = f4{};
+#pragma unroll
+    for (int u = 0; u < kX; ++u) x.load_part(X, ldx, tid, u, first);
+#pragma unroll
+    for (int u = 0; u < kUnits - kX; ++u) y.load_part(Y, ldy, tid, u, first);
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) store(u, 0, lds);
+    if (nk > 1) {
+#pragma unroll
+      for (int u = 0; u < kUnits; ++u) load(u, 1);
+    }
+    __syncthreads();
+    b8 a[2][3], b[BJ][3];
+    auto read_a = [&](const char *s, int i) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        a[i & 1][t] = *reinterpret_cast<const b8 *>(s + ax + i * 256 + t * Tile<TP>::kPlane);
+    };
+    auto read_b = [&](const char *s, int j) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        b[j][t] = *reinterpret_cast<const b8 *>(s + by + j * 256 + t * Tile<TQ>::kPlane);
+    };
+    // Row block i against column blocks j0, j0 + 1: the small products first, from zero.
+    auto pair = [&](int i, int j0, float s) {
+      constexpr int kTa[6] = {2, 0, 1, 1, 0, 0}, kTb[6] = {0, 2, 1, 0, 1, 0};
+      f4 t[2] = {f4{}, f4{}};
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i & 1][kTa[k]], b[j0 + j][kTb[k]], t[j],
+                                                         0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          tot[i][j0 + j][e] = __builtin_fmaf(t[j][e], s, tot[i][j0 + j][e]);
+    };
+    read_a(lds, 0);
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) read_b(lds, j);
+    auto step = [&](int kt, auto more_t) {
+      constexpr bool kMore = decltype(more_t)::value;
+      const char *cur = lds + (kt & 1) * S::kStage;
+      char *nxt = lds + ((kt + 1) & 1) * S::kStage;
+      const float s = ((kt + phase) & 1) ? -1.0f : 1.0f;
+      const int later = min(kt + 2, nk - 1);  // past the end: the last tile again, unused
+#pragma unroll
+      for (int i = 0; i + 1 < BI; ++i) {
+        read_a(cur, i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kMore) {
+#pragma unroll
+          for (int u = 0; u < kUnits; ++u)
+            if (u * (BI - 1) / kUnits == i) {
+              store(u, kt + 1, nxt);
+              load_after(u, later);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < BJ; j += 2) pair(i, j, s);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (kMore) {
+        __syncthreads();
+        read_a(nxt, 0);  // BI is even: the buffer that the last row block does not use
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = 0; j < BJ; j += 2) {
+        pair(BI - 1, j, s);
+        if constexpr (kMore) {
+          __builtin_amdgcn_sched_barrier(0);
+          read_b(nxt, j);
+          read_b(nxt, j + 1);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int kt = 0; kt + 1 < nk; ++kt) step(kt, std::true_type{});
+    step(nk - 1, std::false_type{});
+    f4 z = {};  // x 0 is NaN where an output x is not finite
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z[e] = __builtin_fmaf(tot[i][j][e], 0.0f, z[e]);
+    const bool bad = !((z[0] + z[1]) + (z[2] + z[3]) == 0.0f);
+    if (__any(bad)) fp32(X, ldx, rows_x, Y, ldy, rows_y, R);
+  }
+
+  // The wave's block again with fp32 MFMAs straight from global memory (see "Special
+  // values"): v_mfma_f32_16x16x4f32, lane (g, c) feeding row or column c at reduction step
+  // 4 s + g; sums of 64 steps added into the totals.
+  __device__ __forceinline__ void fp32(const float *X, int64_t ldx, int rows_x, const float *Y,
+                                       int64_t ldy, int rows_y, int R) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = lane & 15, g = lane >> 4;
+    const int pr = (wave / S::WQ) * (16 * BI) + c, qr = (wave % S::WQ) * (16 * BJ) + c;
+    f4 acc[BI][BJ];
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) tot[i][j] = acc[i][j] = f4{};
+    for (int r0 = 0; r0 < R; r0 += 4) {
+      const int64_t r = min(r0 + g, R - 1);
+      const bool in = r0 + g < R;
+      float xv[BI], yv[BJ];
+#pragma unroll
+      for (int i = 0; i < BI; ++i) {
+        const int64_t p = min(pr + 16 * i, rows_x - 1);
+        const float x = XRC ? X[p * ldx + r] : X[r * ldx + p];
+        xv[i] = in ? x : 0.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) {
+        const int64_t q = min(qr + 16 * j, rows_y - 1);
+        const float y = YRC ? Y[q * ldy + r] : Y[r * ldy + q];
+        yv[j] = in ? y : 0.0f;
+      }
+      const bool last = r0 + 4 >= R || (r0 & 63) == 60;
+#pragma unroll
+      for (int i = 0; i < BI; ++i)
+#pragma unroll
+        for (int j = 0; j < BJ; ++j) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[i], yv[j], acc[i][j], 0, 0, 0);
+          if (last) {
+            tot[i][j] += acc[i][j];
+            acc[i][j] = f4{};
+          }
+        }
+    }
+  }
+};
+
+}  // namespace bf3

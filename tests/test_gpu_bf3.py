@@ -1,0 +1,118 @@
+"""Products on the bf16 matrix cores (gemm_bf3.h) against float64: every tile shape at its
+edges, odd sizes and addresses, split reductions, special values, and the mean error."""
+import numpy as np
+import pytest
+
+from conftest import assert_contraction, rand
+from numrs_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def rng():
+    return np.random.default_rng(97)
+
+
+def _at(c, a, off):
+    """`a` on the device `off` floats past a 16-byte boundary."""
+    return c.to_device(np.concatenate([np.zeros(off, np.float32), a.ravel()])).view(off, a.shape)
+
+
+def _product(c, A, B, ta, tb, off=0):
+    M, N = A.shape[1 if ta else 0], B.shape[0 if tb else 1]
+    C = c.to_device(np.full(M * N + off, 7.0, np.float32)).view(off, (M, N))
+    c.matmul(_at(c, A, off), _at(c, B, off), C, trans_a=bool(ta), trans_b=bool(tb))
+    return C.numpy()
+
+
+# Tiles of 64 x 64 ((257, 33, 129): remainders of one row, column and step), with split
+# reductions ((300, 1000, 70), (511, 1000, 513)), 128 x 64 (1001, 777, 1531), 128 x 128
+# (2050, 300, 1030) and 256 x 128 ((2303, 97, 2177), (4097, 40, 1025); one row in the last
+# tile: 4097 takes 256 x 128 only where rows are reduction-contiguous); K = 40 and 33 are two
+# tiles, the first of 8 and of 1 steps; K = 32 and 64 whole tiles.
+SIZES = [(257, 33, 129), (300, 1000, 70), (511, 1000, 513), (1001, 777, 1531), (2050, 300, 1030),
+         (2303, 97, 2177), (4097, 40, 1025), (2048, 32, 2048), (1024, 64, 2048)]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,K,N", SIZES)
+def test_product(hip_ctx, rng, M, K, N, ta, tb):
+    print(f"[gpu] bf3 product {M}x{K}x{N} ta={ta} tb={tb}", flush=True)
+    A, B = rand(rng, (K, M) if ta else (M, K)), rand(rng, (N, K) if tb else (K, N))
+    ref = (A.T if ta else A).astype(np.float64) @ (B.T if tb else B).astype(np.float64)
+    for off in (0, 1):
+        got = _product(hip_ctx, A, B, ta, tb, off)
+        assert_contraction(got, ref, K, what=f"C at {off}")
+        # fp32 sums of 32 steps (six roundings each at most) and of up to 32 such sums
+        # between splits: well under sqrt(K / 32 + 6) units of 2^-24
+        rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert rel < np.sqrt(K / 32 + 6) * 2.0 ** -24, rel
+
+
+@pytest.mark.parametrize("T,fin,fout", [(1000, 617, 1531), (4100, 510, 514), (1537, 65, 2049)])
+def test_linear_pair(hip_ctx, rng, T, fin, fout):
+    """The Linear backward's pair (NN with TN, bias sums) and matmul_backward's (NT with TN) in
+    one grid, at odd sizes; accumulated into what is there."""
+    print(f"[gpu] bf3 pair T={T} in={fin} out={fout}", flush=True)
+    c, lib = hip_ctx, L.load()
+    x, W, g = rand(rng, (T, fin)), rand(rng, (fout, fin)), rand(rng, (T, fout))
+    x64, W64, g64 = (a.astype(np.float64) for a in (x, W, g))
+    dx0, dw0 = rand(rng, (T, fin)), rand(rng, (fout, fin))
+    xd, Wd, gd = (c.to_device(a) for a in (x, W, g))
+    for acc in (0, 1):
+        dx, dw, db = c.to_device(dx0), c.to_device(dw0), c.empty((fout,))
+        assert lib.numrs_hip_linear_backward(c.handle, gd.ptr, xd.ptr, Wd.ptr, dx.ptr, dw.ptr,
+                                             db.ptr, T, fin, fout, acc, acc, 0,
+                                             L.UNBROADCAST_CORRECT) == 0
+        assert_contraction(dx.numpy(), acc * dx0 + g64 @ W64, fout, what="dx")
+        assert_contraction(dw.numpy(), acc * dw0 + g64.T @ x64, T, what="dW")
+        assert_contraction(db.numpy(), g64.sum(0), T, what="db")
+    dA, dB = c.empty((T, fin)), c.empty((fin, fout))
+    Bd = c.to_device(np.ascontiguousarray(W.T))
+    c.matmul_backward(gd, xd, Bd, dA, dB)
+    assert_contraction(dA.numpy(), g64 @ W64, fout, what="dA")
+    assert_contraction(dB.numpy(), x64.T @ g64, T, what="dB")
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_special_values(hip_ctx, rng, ta, tb):
+    """Infinities, NaN, magnitudes above bf16's largest, and rows that only they touch: the
+    values that fp32 products and sums have."""
+    M, K, N = 520, 200, 390
+    A, B = rand(rng, (M, K)), rand(rng, (K, N))
+    A[3, 7], A[100, 0], A[300, 199], A[519, 5] = np.inf, np.nan, -np.inf, 3.4e38
+    A[400, :] = 1e-30
+    A[401, :] = 0.0
+    A[401, 9] = np.inf
+    B[9, 0] = 0.0  # inf * 0
+    B[11, 389] = np.inf
+    B[5, 389] = 0.5  # 3.4e38 times more than 1 overflows in fp32, and inf - inf there is NaN
+    got = _product(hip_ctx, np.ascontiguousarray(A.T) if ta else A,
+                   np.ascontiguousarray(B.T) if tb else B, ta, tb)
+    with np.errstate(all="ignore"):
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+        ref = np.where(np.isfinite(ref) & (np.abs(ref) > np.finfo(np.float32).max),
+                       np.copysign(np.inf, ref), ref)
+    fine = np.isfinite(ref)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    big = np.zeros(ref.shape, bool)
+    big[519] = True  # sums around 3e38: relative only
+    rest = fine & ~big
+    assert_contraction(got[rest], ref[rest], K, what="finite")
+    both = fine & big
+    assert np.all(np.abs(got[both] - ref[both]) <= 1e-6 * np.abs(ref[both]))
+    tiny = np.abs(got[400, fine[400]] - ref[400, fine[400]])
+    assert tiny.max() <= 1e-6 * np.sqrt(K) * 1e-30
+
+
+@pytest.mark.parametrize("K", [64, 512, 2048])
+def test_mean_error(hip_ctx, rng, K):
+    """The matrix unit's sums round down; tiles of alternating sign cancel that.  Without them
+    the mean error is -6e-9 of the rms; the mean of 2^22 errors of 1.5e-7 scatters by 7e-11."""
+    M = N = 2048
+    A, B = rand(rng, (M, K)), rand(rng, (N, K))
+    ref = A.astype(np.float64) @ B.astype(np.float64).T
+    got = _product(hip_ctx, A, B, 0, 1)
+    assert abs((got - ref).mean()) / np.sqrt(np.mean(ref ** 2)) < 1e-9
