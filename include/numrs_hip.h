@@ -308,7 +308,7 @@ int numrs_hip_gemm(numrs_hip_ctx *ctx, const float *A, int64_t lda, const float 
  * Forward: P = softmax(Q K^T / sqrt(D/H)) per (b, h) into P [B*H, S, S],
  * out = P V.  Backward from the saved P: dV = P^T dO, dS = softmax_backward(P,
  * dO V^T), dQ = dS K / sqrt(dh), dK = dS^T Q / sqrt(dh); dq/dk/dv may be NULL;
- * uses B*H*S*S floats of workspace. */
+ * uses up to B*H*S*S floats of the context's memory. */
 int numrs_hip_attention_forward(numrs_hip_ctx *ctx, const float *q, const float *k, const float *v,
                                 float *P, float *out, int64_t B, int64_t S, int64_t H, int64_t D);
 int numrs_hip_attention_backward(numrs_hip_ctx *ctx, const float *q, const float *k,
@@ -328,12 +328,12 @@ int numrs_hip_attention_backward_strided(numrs_hip_ctx *ctx, const float *q, con
                                          float *dv, int64_t B, int64_t S, int64_t H, int64_t D,
                                          int accumulate);
 /* The backward given also the forward's output out (rows at ld_out, like
- * dout), from which the softmax backward's row totals come as dO . O.  For
- * D/H = 64, S = 128 or 256, all three grads non-NULL and accumulate = 0 it
- * runs two kernels: one over query rows (dS = P (dP - dO . O) into a
- * B*H*S*S-float block of the context's memory, and dQ), then one over key
- * rows (dV and dK); every output element is written once, with no atomics.
- * Other calls behave as numrs_hip_attention_backward_strided. */
+ * dout), from which the softmax backward's row totals come as dO . O.  Larger
+ * calls (D/H a multiple of 8 up to 128) run two kernels in both forms: one
+ * over query rows (the row totals, into B*H*S floats of the context's memory,
+ * and dQ), then one over key rows (dV and dK); without out the first walks
+ * the keys once more.  Every output element is written once, with no
+ * atomics. */
 int numrs_hip_attention_backward_out_strided(numrs_hip_ctx *ctx, const float *q, const float *k,
                                              const float *v, int64_t ld_qkv, const float *P,
                                              const float *out, const float *dout, int64_t ld_out,

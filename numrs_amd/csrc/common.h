@@ -287,32 +287,6 @@ int gemm_tn2_colsum(numrs_hip_ctx *ctx, const float *X, int64_t ldx, int64_t M, 
                     const float *Y2, int64_t ldy2, int64_t N2, float *C2, int acc2, float *db,
                     int acc_db, const float *db_part, int64_t db_rows);
 
-
-// One LDS DMA instruction: each lane copies 16 bytes from base + off (off in
-// bytes, per lane; base uniform) into LDS at lds + 16 * lane.  Written as
-// inline asm so that the compiler neither sinks the issue towards the next
-// barrier nor adds its own vmcnt waits for it (it cannot tell which LDS stage
-// an LDS DMA writes, so it would wait for every outstanding one before any
-// fragment read).  The caller places the vmcnt waits: vector-memory
-// operations complete in issue order.  The s_nop covers the M0 write -> LDS
-// DMA hazard.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_dma16(const float *base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(off), "s"(base), "s"(lds)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-
-// s_waitcnt immediate that waits until at most n vector-memory operations
-// are outstanding (expcnt and lgkmcnt left at their no-wait maxima).  The
-// 6-bit vmcnt is split: bits 3:0 of the immediate hold vmcnt[3:0] and bits
-// 15:14 hold vmcnt[5:4].
-constexpr int wait_vm(int n) { return 0x3f70 | (n & 15) | ((n >> 4) << 14); }
-
 }  // namespace numrs_hip
 
 #define NRS_CHECK_CTX(ctx)                       \

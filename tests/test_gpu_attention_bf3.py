@@ -1,0 +1,108 @@
+"""The attention kernels on the bf16 matrix cores (attention_bf3.h) against float64: ragged
+sequences and head sizes, each of their configurations, partial and accumulated gradients, and
+special values."""
+import math
+
+import numpy as np
+import pytest
+
+from conftest import assert_contraction, rand
+from numrs_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+# Each above 2^24 multiply-adds per product and 32 workgroups.  Eight row groups (enough
+# workgroups to fill the chip) or four; sequences below and above 256 (scores kept or formed
+# again); heads of 8 (padded to 32), 24, 40 and 64, 72 (to 96), 128 (the last shape, heads of 96 on part
+# of the chip, keeps the GEMMs); sequences one past, one
+# short of and far from a block's end; 16 x 256 x 8 x 64 is the encoder block's.
+SHAPES = [(4, 130, 8, 40), (16, 129, 16, 8), (2, 300, 16, 32), (8, 257, 12, 72), (32, 100, 16, 24),
+          (3, 520, 30, 128), (10, 255, 10, 96), (5, 321, 7, 64), (16, 256, 8, 64), (4, 383, 24, 64),
+          (2, 300, 16, 96)]
+
+
+def _ref(q, k, v, g, B, S, H):
+    """P, out and the gradients in float64, [B, H, S, .] inside, q's layout outside."""
+    dh = q.shape[1] // H
+    split = lambda a: a.astype(np.float64).reshape(B, S, H, dh).transpose(0, 2, 1, 3)  # noqa: E731
+    merge = lambda a: a.transpose(0, 2, 1, 3).reshape(B * S, H * dh)  # noqa: E731
+    Q, K, V, G = (split(a) for a in (q, k, v, g))
+    s = Q @ K.transpose(0, 1, 3, 2) / math.sqrt(dh)
+    P = np.exp(s - s.max(-1, keepdims=True))
+    P /= P.sum(-1, keepdims=True)
+    dP = G @ V.transpose(0, 1, 3, 2)
+    dS = P * (dP - (dP * P).sum(-1, keepdims=True)) / math.sqrt(dh)
+    return (P.reshape(B * H, S, S), merge(P @ V), merge(dS @ K), merge(dS.transpose(0, 1, 3, 2) @ Q),
+            merge(P.transpose(0, 1, 3, 2) @ G))
+
+
+def _at(a, off):
+    return a.ptr + 4 * off
+
+
+@pytest.mark.parametrize("B,S,H,dh", SHAPES)
+def test_forward_backward(hip_ctx, B, S, H, dh):
+    print(f"[gpu] attention bf3 B={B} S={S} H={H} dh={dh}", flush=True)
+    rng = np.random.default_rng(S * 131 + dh)
+    D, c, lib = H * dh, hip_ctx, L.load()
+    qkv, g, prev = rand(rng, (B * S, 3 * D)), rand(rng, (B * S, D)), rand(rng, (B * S, 3 * D))
+    q, k, v = qkv[:, :D], qkv[:, D:2 * D], qkv[:, 2 * D:]
+    P64, out64, *grads = _ref(q, k, v, g, B, S, H)
+    ref = np.concatenate(grads, axis=1)
+    x, gd = c.to_device(qkv), c.to_device(g)
+    P, out = c.to_device(np.full((B * H, S, S), np.nan, np.float32)), c.empty((B * S, D))
+    qp, kp, vp = x.ptr, _at(x, D), _at(x, 2 * D)
+    assert lib.numrs_hip_attention_forward_strided(c.handle, qp, kp, vp, 3 * D, P.ptr, out.ptr, D,
+                                                   B, S, H, D) == 0
+    assert_contraction(P.numpy(), P64, dh, what="P")
+    assert_contraction(out.numpy(), out64, S, what="out")
+    for what, given, acc, keep in (("out", True, 0, (1, 1, 1)), ("no out", False, 0, (1, 1, 1)),
+                                   ("acc", True, 1, (1, 1, 1)), ("dq", True, 0, (1, 0, 0)),
+                                   ("dk", False, 1, (0, 1, 0)), ("dk dv", True, 0, (0, 1, 1))):
+        d = c.to_device(prev)
+        ptrs = [p if want else None for p, want in zip((d.ptr, _at(d, D), _at(d, 2 * D)), keep)]
+        if given:
+            rc = lib.numrs_hip_attention_backward_out_strided(
+                c.handle, qp, kp, vp, 3 * D, P.ptr, out.ptr, gd.ptr, D, *ptrs, B, S, H, D, acc)
+        else:
+            rc = lib.numrs_hip_attention_backward_strided(
+                c.handle, qp, kp, vp, 3 * D, P.ptr, gd.ptr, D, *ptrs, B, S, H, D, acc)
+        assert rc == 0
+        got = d.numpy()
+        for i, want in enumerate(keep):
+            sl = slice(i * D, (i + 1) * D)
+            if want:
+                assert_contraction(got[:, sl], acc * prev[:, sl] + ref[:, sl], S + dh,
+                                   what=f"{what}: d{'qkv'[i]}")
+            else:
+                assert np.array_equal(got[:, sl], prev[:, sl]), f"{what}: d{'qkv'[i]} touched"
+
+
+@pytest.mark.parametrize("B,S,H,dh", [(16, 200, 16, 64), (2, 300, 16, 64)])
+def test_special_values(hip_ctx, B, S, H, dh):
+    """An infinite key element (scores of +-inf: NaN rows, or probabilities of 0), an infinite
+    value and magnitudes above bf16's largest: what fp32 products give."""
+    rng = np.random.default_rng(5)
+    D, c, lib = H * dh, hip_ctx, L.load()
+    q, k, v, g = (rand(rng, (B * S, D)) for _ in range(4))
+    k[7, 3] = np.inf         # head 0 of sequence 0: +inf or -inf scores by the sign of q[., 3]
+    v[S + 9, dh + 1] = np.inf  # head 1 of sequence 1: its output column
+    k[20, 2 * dh + 2] = 3.4e38
+    q[20, 2 * dh + 2] = 0.0  # a score of 0 from it; the others overflow
+    with np.errstate(all="ignore"):
+        P64, out64, *_ = _ref(q, k, v, g, B, S, H)
+    dev = [c.to_device(a) for a in (q, k, v)]
+    P, out = c.empty((B * H, S, S)), c.empty((B * S, D))
+    assert lib.numrs_hip_attention_forward(c.handle, *(a.ptr for a in dev), P.ptr, out.ptr, B, S, H, D) == 0
+    p, o = P.numpy(), out.numpy()
+    head = 2  # k = 3.4e38 times a q above 1 overflows in fp32 and not in float64
+    ok = np.arange(B * H) != head
+    assert np.array_equal(np.isnan(p[ok]), np.isnan(P64[ok]))
+    assert_contraction(np.nan_to_num(p[ok]), np.nan_to_num(P64[ok]), dh, what="P")
+    cols = np.ones((B * S, D), bool)
+    cols[:S, head * dh:(head + 1) * dh] = False
+    assert np.array_equal(np.isnan(o[cols]), np.isnan(out64[cols]))
+    assert np.array_equal(np.isposinf(o[cols]), np.isposinf(out64[cols]))
+    fine = cols & np.isfinite(out64)
+    assert_contraction(o[fine], out64[fine], S, what="out")
+    assert np.isfinite(p[head, 20]).all() and abs(p[head, 20].sum() - 1) < 1e-5
