@@ -189,7 +189,7 @@ int numrs_hip_graph_launch(numrs_hip_graph *g);
 int numrs_hip_graph_destroy(numrs_hip_graph *g);
 
 /* ---------------------------------------------------------------------- */
-/* Dense contractions (fp32 MFMA)                                          */
+/* Dense contractions (fp32, on the matrix cores)                          */
 /* ---------------------------------------------------------------------- */
 
 /* matmul_backward (autograd/backward.rs:113-149) for C[M,N] = A[M,K] @ B[K,N]:
