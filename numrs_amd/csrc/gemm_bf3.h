@@ -92,17 +92,20 @@ struct Loader {
     const int u = tid + NT * i;
     return RC ? u % kChunks : u / EXT;
   }
+  // The row that unit i reads, of `rows` that exist.
+  static __device__ __forceinline__ int read_row(int tid, int i, int rows) {
+    return kPairs ? min(row(tid, 0), rows - 2) + i : min(row(tid, i), rows - 1);
+  }
   // rows: how many of the tile's rows exist; at least 1, pairs: 2 (pairs_fit).  A pair whose
   // first row is an odd last one reads the row before and that one, and trades places.
   __device__ __forceinline__ void init(int tid, int64_t ld, int rows) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      int r = row(tid, i);
+      const int r = row(tid, i), from = read_row(tid, i, rows);
       const int ch = chunk(tid, i);
       const int put = kPairs && r - i > rows - 2 ? r ^ 1 : r;
       slot[i] = ch * Tile<EXT>::kChunkStride + (put ^ swizzle(ch)) * 16;
-      r = kPairs ? min(r - i, rows - 2) + i : min(r, rows - 1);
-      off[i] = RC ? (Off)((Off)r * (Off)ld + (Off)(8 * ch)) : (Off)r;
+      off[i] = RC ? (Off)((Off)from * (Off)ld + (Off)(8 * ch)) : (Off)from;
     }
   }
   // Unit i (pairs: both at i = 0) of the whole tile at `base`, row 0 of the tile at its first
@@ -140,6 +143,9 @@ struct Loader {
       v[i][j] = in ? x : 0.0f;
     }
   }
+  __device__ __forceinline__ float sum(int i) const {
+    return ((v[i][0] + v[i][1]) + (v[i][2] + v[i][3])) + ((v[i][4] + v[i][5]) + (v[i][6] + v[i][7]));
+  }
   // sign: 0, or the sign bit for the terms of -x (SIGNED).
   template <bool SIGNED>
   __device__ __forceinline__ void store(char *lds, int i, uint32_t sign) const {
@@ -175,11 +181,13 @@ struct Shape {
   }
 };
 
-template <bool XRC, bool YRC, class S>
+template <bool XRC, bool YRC, class S, bool SUMS = false>
 struct Product {
   static constexpr int BI = S::BI, BJ = S::BJ, TP = S::TP, TQ = S::TQ, NT = S::NT;
   static_assert(BI % 2 == 0 && BJ % 2 == 0, "block pairs");
+  using LX = Loader<XRC, TP, NT, S::WIDE>;
   f4 tot[BI][BJ];
+  float rowsum[SUMS ? LX::N : 1];  // SUMS: the sums of the rows of X that the thread's units read
 
   // tot = X Y over R >= 1 reduction steps; X: row 0 of the tile at the first step, rows_x of
   // its TP rows exist (Y alike).  lds: S::kLds bytes.
@@ -198,7 +206,6 @@ struct Product {
   // row block of this one, so the last phase's MFMAs cover the first reads of the next stage.
   __device__ __forceinline__ void run(const float *X, int64_t ldx, int rows_x, const float *Y,
                                       int64_t ldy, int rows_y, int R, int phase, char *lds) {
-    using LX = Loader<XRC, TP, NT, S::WIDE>;
     using LY = Loader<YRC, TQ, NT, S::WIDE>;
     constexpr int kX = LX::N, kUnits = LX::N + LY::N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -220,11 +227,16 @@ struct Product {
       else
         y.load(Y + r * ystep, ldy, tid, u - kX);
     };
+    float part[kX] = {};  // SUMS: of up to 16 tiles
+    if constexpr (SUMS)
+#pragma unroll
+      for (int u = 0; u < kX; ++u) rowsum[u] = 0.0f;
     // Unit u of tile kt, whose Y is negated when kt + phase is odd.
     auto store = [&](int u, int kt, char *s) {
-      if (u < kX)
+      if (u < kX) {
         x.template store<false>(s, u, 0);
-      else
+        if constexpr (SUMS) part[u] += x.sum(u);
+      } else
         y.template store<true>(s + Tile<TP>::kBytes, u - kX, (uint32_t)(kt + phase) << 31);
     };
     // Unit u's registers are free for its next load once the units it loads with are stored.
@@ -320,7 +332,16 @@ struct Product {
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    for (int kt = 0; kt + 1 < nk; ++kt) step(kt, std::true_type{});
+    for (int kt = 0; kt + 1 < nk; ++kt) {
+      step(kt, std::true_type{});
+      if constexpr (SUMS)
+        if ((kt & 15) == 14)
+#pragma unroll
+          for (int u = 0; u < kX; ++u) rowsum[u] += part[u], part[u] = 0.0f;
+    }
+    if constexpr (SUMS)
+#pragma unroll
+      for (int u = 0; u < kX; ++u) rowsum[u] += part[u];
     step(nk - 1, std::false_type{});
     f4 z = {};  // x 0 is NaN where an output x is not finite
 #pragma unroll

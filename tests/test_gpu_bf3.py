@@ -75,6 +75,36 @@ def test_linear_pair(hip_ctx, rng, T, fin, fout):
     assert_contraction(dB.numpy(), x64.T @ g64, T, what="dB")
 
 
+@pytest.mark.parametrize("T,fin,fout", [(300, 257, 300), (1000, 617, 1531), (8193, 130, 513),
+                                        (4096, 512, 2048), (2100, 2050, 2305)])
+@pytest.mark.parametrize("off,acc", [(0, 0), (1, 1)])
+def test_bias_sums(hip_ctx, rng, T, fin, fout, off, acc):
+    """A Linear's bias gradient, formed by the dW product's own tiles: every tile shape, odd last
+    rows, split and whole reductions, accumulated, db at any address, values that are not finite."""
+    print(f"[gpu] bf3 bias sums T={T} in={fin} out={fout} off={off} acc={acc}", flush=True)
+    c, lib = hip_ctx, L.load()
+    x, W, g, db0 = rand(rng, (T, fin)), rand(rng, (fout, fin)), rand(rng, (T, fout)), rand(rng, (fout,))
+    xd, Wd, dx, dw = c.to_device(x), c.to_device(W), c.empty((T, fin)), c.empty((fout, fin))
+
+    def run():
+        db, gd = _at(c, db0, off), c.to_device(g)
+        assert lib.numrs_hip_linear_backward(c.handle, gd.ptr, xd.ptr, Wd.ptr, dx.ptr, dw.ptr, db.ptr,
+                                             T, fin, fout, 0, 0, acc, L.UNBROADCAST_CORRECT) == 0
+        return db.numpy()
+
+    got, ref = run(), acc * db0 + g.astype(np.float64).sum(0)
+    # three roundings of eight steps, up to 16 tiles a partial sum, T / 512 of those, two of the
+    # four threads', up to 32 splits' and db0's
+    rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert rel < np.sqrt(3 + 16 + T / 512 + 2 + 32 + 1) * 2.0 ** -24, rel
+    assert np.array_equal(got, run())
+    g[T - 1, 0], g[5, fout - 1], g[0, 7] = np.inf, np.nan, -np.inf
+    bad = run()
+    assert bad[0] == np.inf and np.isnan(bad[-1]) and bad[7] == -np.inf
+    rest = np.setdiff1d(np.arange(fout), [0, 7, fout - 1])
+    assert np.array_equal(bad[rest], got[rest])
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_special_values(hip_ctx, rng, ta, tb):
     """Infinities, NaN, magnitudes above bf16's largest, and rows that only they touch: the
