@@ -108,8 +108,8 @@ struct SplitSet {
 };
 
 // Column sums out[c] (+)= sum_r g[r ldg + c] of a [rows, cols] block in one
-// pass (the Linear backward's bias gradient, carried by the launch that
-// reduces the weight gradient's splits).  A workgroup owns eight columns
+// pass, carried by the launch that reduces a product's splits or on their own
+// (a bias gradient where its Linear has no dx or no dW, or an LSTM layer's).  A workgroup owns eight columns
 // (two float4 groups; cols % 4 == 0, a last group past the end is skipped)
 // and 128 row classes: thread k reads chunk k % 2 of rows k / 2, k / 2 + 128,
 // ... and adds them in order, 16 loads in flight; the 128 class sums of a
