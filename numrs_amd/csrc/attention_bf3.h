@@ -346,15 +346,27 @@ struct Scale {
 // Running maximum and sum of 2^score of one lane's keys.
 struct RowStat {
   float m = -INFINITY, l = 0.0f;
-  // Keys key0 + 16 k + e, those from S on left out (WHOLE: there are none).
+  // Keys key0 + 16 k + e, those from S on left out (WHOLE: there are none).  INF, the pass whose
+  // result stands: a NaN score makes the row's sum NaN, also where fmaxf drops it because the
+  // lane has no other key yet.  (In the other form such a key's own probability is NaN, and with
+  // it the row's output, which calls for this pass.)
   template <bool INF, bool WHOLE, int N>
   __device__ __forceinline__ void add(const f4 (&y)[N], const Scale &sc, int key0, int S) {
     float top = -INFINITY;
+    bool nan = false;
 #pragma unroll
     for (int k = 0; k < N; ++k)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (WHOLE || key0 + 16 * k + e < S) top = fmaxf(top, y[k][e]);
+        if (WHOLE || key0 + 16 * k + e < S) {
+          top = fmaxf(top, y[k][e]);
+          nan = nan || y[k][e] != y[k][e];
+        }
+    if (INF && nan) {
+      l = NAN;
+      m = fmaxf(m, 0.0f);  // not -inf: part() keeps l
+      return;
+    }
     top = fmaxf(m, top * sc.hi);
     if (top == -INFINITY) return;  // no key of this lane yet
     l = l * __builtin_amdgcn_exp2f(m - top);

@@ -106,3 +106,27 @@ def test_special_values(hip_ctx, B, S, H, dh):
     fine = cols & np.isfinite(out64)
     assert_contraction(o[fine], out64[fine], S, what="out")
     assert np.isfinite(p[head, 20]).all() and abs(p[head, 20].sum() - 1) < 1e-5
+
+
+@pytest.mark.parametrize("B,S,H,dh", [(16, 200, 16, 64), (2, 300, 16, 64)])
+def test_nan_keys(hip_ctx, B, S, H, dh):
+    """NaN keys that fill one lane's four first keys, or a later group of four, or sit beside a
+    finite one: every probability of the head's rows is NaN, and no other head's is."""
+    rng = np.random.default_rng(6)
+    D, c, lib = H * dh, hip_ctx, L.load()
+    q, k, v = (rand(rng, (B * S, D)) for _ in range(3))
+    heads = {0: slice(0, 4), 1: slice(4, 8), 2: slice(8, 12), 3: slice(12, 16), 4: slice(0, 16),
+             5: slice(20, 24), 6: slice(2, 3), 7: slice(0, S), 8: slice(S - 1, S)}
+    for h, rows in heads.items():
+        k[rows, h * dh + 5] = np.nan
+    k[S:S + 4, 5] = np.inf  # head 0 of sequence 1: scores of +inf or -inf, by the sign of q
+    P, out = c.empty((B * H, S, S)), c.empty((B * S, D))
+    dev = [c.to_device(a) for a in (q, k, v)]
+    assert lib.numrs_hip_attention_forward(c.handle, *(a.ptr for a in dev), P.ptr, out.ptr, B, S, H, D) == 0
+    p, o = P.numpy(), out.numpy()
+    want = np.zeros(p.shape, bool)
+    want[list(heads)] = True
+    want[H] = (q[S:2 * S, 5] > 0)[:, None]  # inf - inf in those rows
+    assert np.array_equal(np.isnan(p), want)
+    assert np.array_equal(np.isnan(o.reshape(B, S, H, dh).transpose(0, 2, 1, 3)).reshape(B * H, S, dh),
+                          np.broadcast_to(want[:, :, :1], (B * H, S, dh)))
