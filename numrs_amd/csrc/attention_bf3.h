@@ -24,6 +24,8 @@ namespace attn {
 using bf3::b8;
 using bf3::f4;
 using bf3::f4u;
+using bf3::kScale;
+using bf3::kUnscale;
 using bf3::u4;
 
 // NW x NG waves: wave w owns rows 16 (w % NW) .. + 15 of the workgroup's 16 NW against part
@@ -42,6 +44,7 @@ struct Cfg {
   static constexpr bool parts_fit(int images) { return (NG - 1) * NW * 64 * NB * 16 <= images * kImage; }
 };
 
+// The terms of operands, which come multiplied by kScale (products: times kUnscale).
 __device__ __forceinline__ void split8(const float (&v)[8], u4 &h, u4 &m, u4 &l) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -131,8 +134,11 @@ struct Block {
       constexpr int kRow = TR ? C::DH : C::BLK;
       const int slot = TR ? u % C::DH : u / (C::DH / 8), ch = TR ? u / C::DH : u % (C::DH / 8);
       char *p = lds + ((int64_t)ch * kRow + (slot ^ bf3::swizzle(ch & 3))) * 16;
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = v[i][j] * kScale;
       u4 h, m, l;
-      split8(v[i], h, m, l);
+      split8(x, h, m, l);
       if (!in[i]) h = m = l = u4{};  // a column past the head's last
       *reinterpret_cast<u4 *>(p) = h;
       *reinterpret_cast<u4 *>(p + C::kPlane) = m;
@@ -151,7 +157,7 @@ __device__ __forceinline__ void frag(Terms &f, const char *lds, int step, int sl
 }
 
 // The wave's own rows as second operand: lane (g, c) holds row `row`, columns 32 s + 8 g .. + 7;
-// odd steps negated (blocks32 subtracts them).
+// times kScale, odd steps negated (blocks32 subtracts them).
 template <class C>
 __device__ __forceinline__ void own_rows(Terms (&f)[C::NS], const float *row, int dh, int g) {
 #pragma unroll
@@ -160,18 +166,19 @@ __device__ __forceinline__ void own_rows(Terms (&f)[C::NS], const float *row, in
     const bool in = at < dh;
     const float *p = row + (in ? at : 0);
     const f4u a = *reinterpret_cast<const f4u *>(p), b = *reinterpret_cast<const f4u *>(p + 4);
+    const float scale = (s & 1) ? -kScale : kScale;
     float v[8];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      v[j] = in ? ((s & 1) ? -a[j] : a[j]) : 0.0f;
-      v[4 + j] = in ? ((s & 1) ? -b[j] : b[j]) : 0.0f;
+      v[j] = in ? scale * a[j] : 0.0f;
+      v[4 + j] = in ? scale * b[j] : 0.0f;
     }
     f[s].set(v);
   }
 }
 
-// y[u]: the staged rows 16 (k + u) + 4 g + e against the wave's row c, u = 0, 1.  Steps
-// alternate in sign: the MFMA's sums round down (gemm_bf3.h).
+// y[u] kUnscale: the staged rows 16 (k + u) + 4 g + e against the wave's row c, u = 0, 1.
+// Steps alternate in sign: the MFMA's sums round down (gemm_bf3.h).
 template <class C>
 __device__ __forceinline__ void blocks32(f4 (&y)[2], const char *lds, int k, const Terms (&own)[C::NS], int c,
                                          int g) {
@@ -199,7 +206,8 @@ __device__ __forceinline__ void blocks32(f4 (&y)[2], const char *lds, int k, con
   for (int u = 0; u < 2; ++u) y[u] -= odd[u];
 }
 
-// acc[b] += sign (the image's columns 16 b + 4 g + e) of 32 staged rows times the wave's values p.
+// acc[b] += sign (the image's columns 16 b + 4 g + e) of 32 staged rows times the wave's values p
+// (times kScale).
 template <class C>
 __device__ __forceinline__ void rows32(f4 (&acc)[C::NB], const char *lds, int grp, const Terms &p,
                                        float sign, int c, int g) {
@@ -214,7 +222,7 @@ __device__ __forceinline__ void rows32(f4 (&acc)[C::NB], const char *lds, int gr
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[b + u][e] = __builtin_fmaf(t[u][e], sign, acc[b + u][e]);
+      for (int e = 0; e < 4; ++e) acc[b + u][e] = __builtin_fmaf(t[u][e], sign * kUnscale, acc[b + u][e]);
   }
 }
 
@@ -438,6 +446,7 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(const float *q, const float 
   vb.init(ld, dh, tid);
   const int nb = (S + C::BLK - 1) / C::BLK;
   RowStat st;
+  const Scale sf{sc.hi * kUnscale, sc.lo * kUnscale};  // of blocks32's scores
   f4 kept[KEEP > 0 ? KEEP : 1][N16];
   // The wave's first key of block i, and whether all of its keys there exist.
   auto first = [&](int i) { return i * C::BLK + grp * C::SUB; };
@@ -450,9 +459,9 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(const float *q, const float 
       y[n] = t[0], y[n + 1] = t[1];
     }
     if (whole(i))
-      st.add<false, true>(y, sc, first(i) + 4 * g, S);
+      st.add<false, true>(y, sf, first(i) + 4 * g, S);
     else
-      st.add<false, false>(y, sc, first(i) + 4 * g, S);
+      st.add<false, false>(y, sf, first(i) + 4 * g, S);
   };
   auto load_k = [&](int i) { kb.load(k, ld, i * C::BLK, S, tid); };
   walk<KEEP>(nb, load_k, [&]() { kb.store(kl, tid); }, [&](int i) {
@@ -481,9 +490,9 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(const float *q, const float 
       f4u w;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        w[e] = __builtin_amdgcn_exp2f(sc.at<false>(y[u][e], st.m)) * inv;
+        w[e] = __builtin_amdgcn_exp2f(sf.at<false>(y[u][e], st.m)) * inv;
         if (!WHOLE && key + e >= S) w[e] = 0.0f;
-        p[4 * u + e] = sign * w[e];
+        p[4 * u + e] = sign * kScale * w[e];
       }
       if (live && (WHOLE || key + 4 <= S))
         *reinterpret_cast<f4u *>(Pr + key) = w;
@@ -617,7 +626,7 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
           }
           d += part;
         });
-    d = rows4(d, [](float a, float b) { return a + b; });
+    d = rows4(d, [](float a, float b) { return a + b; }) * kUnscale;
     const int r = wave % C::NW * 16 + c;
     if (g == 0) total[grp * 16 * C::NW + r] = d;
     __syncthreads();
@@ -659,7 +668,8 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ds[4 * u + e] = sign * (p[n + u][e] * (dp[u][e] - d));
+            for (int e = 0; e < 4; ++e)
+              ds[4 * u + e] = sign * kScale * (p[n + u][e] * __builtin_fmaf(dp[u][e], kUnscale, -d));
           Terms t;
           t.set(ds);
           rows32<C>(acc, kl, (n0 + n) / 2, t, sign, c, g);
@@ -760,8 +770,8 @@ __global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const fl
           for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              pv[4 * u + e] = sign * p[n + u][e];
-              ds[4 * u + e] = sign * (p[n + u][e] * (dp[u][e] - d[n + u][e]));
+              pv[4 * u + e] = sign * kScale * p[n + u][e];
+              ds[4 * u + e] = sign * kScale * (p[n + u][e] * __builtin_fmaf(dp[u][e], kUnscale, -d[n + u][e]));
             }
           Terms t;
           t.set(pv);

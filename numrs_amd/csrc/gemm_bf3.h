@@ -1,10 +1,15 @@
 // Products of fp32 matrices on the bf16 matrix cores, at fp32 accuracy.
 //
-// An fp32 value is the sum of three bf16 values, x = h + m + l with h = bf16(x),
+// An fp32 value is the sum of three bf16 values (Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 artificial intelligence datatype for higher-precision computations", ARITH 2019),
+// x = h + m + l with h = bf16(x),
 // m = bf16(x - h), l = x - h - m (round to nearest even; both differences are exact, and
-// what is left after two roundings fits bf16's 8 bits).  A product is then
+// what is left after two roundings fits bf16's 8 bits).  Operands are split times 2^16, and
+// the sums multiplied by 2^-32: every fp32 value, the subnormal ones too, is then a multiple
+// of bf16's smallest subnormal, 2^-133, and the split exact (conversion and MFMA keep bf16
+// subnormals: measured).  A product is
 //   x y = hx hy + (hx my + mx hy) + (mx my + hx ly + lx hy) + [mx ly + lx my + lx ly],
-// the bracket, at most 2^-26 |x y|, left out: six v_mfma_f32_16x16x32_bf16 per 16 x 16 x 32
+// the bracket, at most 2^-24 |x y|, left out: six v_mfma_f32_16x16x32_bf16 per 16 x 16 x 32
 // block, accumulated in fp32, smallest terms first, from zero for every 32 reduction steps;
 // the sums of 32 steps are added into fp32 totals.  Measured against float64 on N(0, 1)
 // operands, relative 2-norm error at R = 256 | 512 | 2048 reduction steps: 0.7 | 0.9 |
@@ -17,11 +22,10 @@
 // of bf16 (hipBLASLt's plain bf16 product of that size: 1.14; the fp32 MFMA kernel that
 // this replaced: 142 TFLOP/s).
 //
-// Special values.  An infinity, a NaN or a magnitude above bf16's largest finite value has
-// a term x - h that is not finite, and makes every output of its row or column NaN or
-// infinite.  A wave that finds such an output recomputes its block with fp32 MFMAs, so
-// that the results are those of fp32 arithmetic.  Below 2^-110 the terms m and l lose bits
-// to bf16's smallest subnormal, 2^-133: an absolute error of at most 2^-134 per operand.
+// Special values.  An infinity, a NaN or a magnitude of 2^112 or more has a term x - h that
+// is not finite, and makes every output of its row or column NaN or infinite; so does a sum
+// of 32 products of 2^96 or more its output.  A wave that finds such an output recomputes
+// its block with fp32 MFMAs, so that the results are those of fp32 arithmetic.
 #pragma once
 
 #include <type_traits>
@@ -51,6 +55,8 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t &h, uint32_t &
   m = pack(ra, rb);
   l = pack(ra - lo(m), rb - hi(m));
 }
+
+constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;  // of operands, and back for their products
 
 constexpr int kBR = 32;           // reduction steps per tile (one MFMA's)
 constexpr int kChunks = kBR / 8;  // 16-byte chunks (8 bf16) of a row
@@ -146,17 +152,13 @@ struct Loader {
   __device__ __forceinline__ float sum(int i) const {
     return ((v[i][0] + v[i][1]) + (v[i][2] + v[i][3])) + ((v[i][4] + v[i][5]) + (v[i][6] + v[i][7]));
   }
-  // sign: 0, or the sign bit for the terms of -x (SIGNED).
-  template <bool SIGNED>
-  __device__ __forceinline__ void store(char *lds, int i, uint32_t sign) const {
-    auto at = [&](int j) {
-      return SIGNED ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i][j]) ^ sign) : v[i][j];
-    };
+  // The terms of the values times `scale`: kScale or -kScale.
+  __device__ __forceinline__ void store(char *lds, int i, float scale) const {
     u4 h, m, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       uint32_t a, b, c;
-      split2(at(2 * j), at(2 * j + 1), a, b, c);
+      split2(v[i][2 * j] * scale, v[i][2 * j + 1] * scale, a, b, c);
       h[j] = a, m[j] = b, l[j] = c;
     }
     char *p = lds + slot[i];
@@ -234,10 +236,10 @@ struct Product {
     // Unit u of tile kt, whose Y is negated when kt + phase is odd.
     auto store = [&](int u, int kt, char *s) {
       if (u < kX) {
-        x.template store<false>(s, u, 0);
+        x.store(s, u, kScale);
         if constexpr (SUMS) part[u] += x.sum(u);
       } else
-        y.template store<true>(s + Tile<TP>::kBytes, u - kX, (uint32_t)(kt + phase) << 31);
+        y.store(s + Tile<TP>::kBytes, u - kX, ((kt + phase) & 1) ? -kScale : kScale);
     };
     // Unit u's registers are free for its next load once the units it loads with are stored.
     auto load_after = [&](int u, int kt) {
@@ -298,7 +300,7 @@ struct Product {
       constexpr bool kMore = decltype(more_t)::value;
       const char *cur = lds + (kt & 1) * S::kStage;
       char *nxt = lds + ((kt + 1) & 1) * S::kStage;
-      const float s = ((kt + phase) & 1) ? -1.0f : 1.0f;
+      const float s = ((kt + phase) & 1) ? -kUnscale : kUnscale;
       const int later = min(kt + 2, nk - 1);  // past the end: the last tile again, unused
 #pragma unroll
       for (int i = 0; i + 1 < BI; ++i) {

@@ -130,3 +130,46 @@ def test_nan_keys(hip_ctx, B, S, H, dh):
     assert np.array_equal(np.isnan(p), want)
     assert np.array_equal(np.isnan(o.reshape(B, S, H, dh).transpose(0, 2, 1, 3)).reshape(B * H, S, dh),
                           np.broadcast_to(want[:, :, :1], (B * H, S, dh)))
+
+
+@pytest.mark.parametrize("B,S,H,dh", [(16, 200, 16, 64), (2, 300, 16, 64)])
+@pytest.mark.parametrize("given", [True, False])
+def test_small_values(hip_ctx, B, S, H, dh, given):
+    """Values, output gradients and probabilities near the end of fp32's range: the products
+    have the relative error of ordinary ones (some 3e-7 of sums of 300 terms; the reference is
+    formed of the probabilities that the forward left)."""
+    rng = np.random.default_rng(8)
+    D, c, lib = H * dh, hip_ctx, L.load()
+    q, k = rand(rng, (B * S, D), 1e10), rand(rng, (B * S, D), 1e-10)
+    v, g = rand(rng, (B * S, D)), rand(rng, (B * S, D), 1e-34)
+    q[:, 0], k[:, 0] = 1e10, 0.0
+    k[3::50, 0] = -6e-8  # head 0: scores of -75 at these keys, probabilities of 1e-35
+    g[:, :dh] *= 1e30    # head 0: larger gradients
+    split = lambda a: a.astype(np.float64).reshape(B, S, H, dh).transpose(0, 2, 1, 3)  # noqa: E731
+    rel = lambda got, ref: np.linalg.norm(got - ref) / np.linalg.norm(ref)  # noqa: E731
+    for scale in (1.0, 1e-37):
+        vs = v * np.float32(scale)
+        qd, kd, vd, gd = (c.to_device(a) for a in (q, k, vs, g))
+        P, out, dq, dk, dv = c.empty((B * H, S, S)), *(c.empty((B * S, D)) for _ in range(4))
+        assert lib.numrs_hip_attention_forward(c.handle, qd.ptr, kd.ptr, vd.ptr, P.ptr, out.ptr, B, S, H, D) == 0
+        if given:
+            rc = lib.numrs_hip_attention_backward_out_strided(
+                c.handle, qd.ptr, kd.ptr, vd.ptr, D, P.ptr, out.ptr, gd.ptr, D, dq.ptr, dk.ptr, dv.ptr, B, S, H, D, 0)
+        else:
+            rc = lib.numrs_hip_attention_backward(c.handle, qd.ptr, kd.ptr, vd.ptr, P.ptr, gd.ptr, dq.ptr, dk.ptr,
+                                                  dv.ptr, B, S, H, D, 0)
+        assert rc == 0
+        p = P.numpy().astype(np.float64).reshape(B, H, S, S)
+        Q, V, G = split(q), split(vs), split(g)
+        assert rel(split(out.numpy()), p @ V) < 1e-6
+        dV, dV64 = split(dv.numpy()), p.transpose(0, 1, 3, 2) @ G
+        few = np.isin((np.arange(B * S).reshape(B, S) - 3) % 50, 0)  # [B, S]
+        for b in range(B):
+            assert 0 < p[b, 0][:, few[b]].max() < 1e-33
+            assert rel(dV[b, 0, few[b]], dV64[b, 0, few[b]]) < 1e-6
+        assert rel(dV[:, 1:], dV64[:, 1:]) < 1e-6
+        if scale == 1.0:  # else dO V^T is below fp32's range
+            dP = G @ V.transpose(0, 1, 3, 2)
+            dS = p * (dP - (dP * p).sum(-1, keepdims=True)) / math.sqrt(dh)
+            # dP - D cancels: errors of 5e-7 of dP's size, not of the difference's
+            assert rel(split(dk.numpy())[:, 1:], (dS.transpose(0, 1, 3, 2) @ Q)[:, 1:]) < 4e-6

@@ -146,3 +146,31 @@ def test_mean_error(hip_ctx, rng, K):
     ref = A.astype(np.float64) @ B.astype(np.float64).T
     got = _product(hip_ctx, A, B, 0, 1)
     assert abs((got - ref).mean()) / np.sqrt(np.mean(ref ** 2)) < 1e-9
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("a,b", [(1e-37, 1e10), (1e10, 3e-38), (1e-40, 1e30), (2e-36, 0.5), (1e-20, 1e-17),
+                                 (1e20, 1e7), (1e30, 1e-36), (1e35, 1e-3)])
+def test_small_and_large_operands(hip_ctx, rng, ta, tb, a, b):
+    """Operands far from 1, down to fp32's subnormals and up to sums just under 2^96: the error
+    relative to the result is that of ordinary operands (test_product).  Above 2^112 the fp32
+    MFMAs' sums of 64 steps, twice that (measured for them: 1.9e-7)."""
+    M, K, N = 520, 333, 390
+    A, B = rand(rng, (M, K), a), rand(rng, (K, N), b)
+    got = _product(hip_ctx, np.ascontiguousarray(A.T) if ta else A,
+                   np.ascontiguousarray(B.T) if tb else B, ta, tb)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    # results below 2^-126 are rounded to multiples of 2^-149
+    least = np.sqrt(ref.size) * 2.0 ** -150 / np.linalg.norm(ref)
+    assert rel < (2 if a > 1e33 else 1) * np.sqrt(K / 32 + 6) * 2.0 ** -24 + least, rel
+
+
+def test_left_out_terms(hip_ctx):
+    """Operands whose left-out products are the largest, 2^-24 of each product and of one sign:
+    the result is off by that and no more."""
+    M, K, N = 520, 256, 390
+    x = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)  # h = 1, m = 2^-8, l = -2^-17
+    got = _product(hip_ctx, np.full((M, K), x), np.full((K, N), x), 0, 0)
+    ref = K * float(x) ** 2
+    assert np.abs(got / ref - 1).max() < (1.01 + np.sqrt(K / 32 + 6)) * 2.0 ** -24
