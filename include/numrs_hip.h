@@ -191,6 +191,10 @@ int numrs_hip_graph_destroy(numrs_hip_graph *g);
 /* ---------------------------------------------------------------------- */
 /* Dense contractions (fp32, on the matrix cores)                          */
 /* ---------------------------------------------------------------------- */
+/* Products above 2^24 multiply-adds, and attention, run on the bf16 matrix
+ * cores from exact three-term splits of the fp32 operands; outputs touched by
+ * an infinity, a NaN or a magnitude of 2^112 or more are formed again with
+ * fp32 products: the same results as fp32 arithmetic gives, in more time. */
 
 /* matmul_backward (autograd/backward.rs:113-149) for C[M,N] = A[M,K] @ B[K,N]:
  *   dA[M,K] = dC @ B^T,  dB[K,N] = A^T @ dC.

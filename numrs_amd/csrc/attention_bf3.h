@@ -264,30 +264,77 @@ __device__ __forceinline__ void store_rows(float *row, const f4 (&acc)[C::NB], f
     }
 }
 
-// fp32 forms of blocks32 and rows32 from global memory (non-finite values, see gemm_bf3.h):
-// rows r0 + 4 g + e of `x` against the wave's row `own`, and their columns times p.
-__device__ __forceinline__ f4 block16_fp32(const float *x, int64_t ld, int r0, int n, const float *own,
-                                           int dh, int c, int g) {
-  f4 t = {};
-  const float *xr = x + (int64_t)min(r0 + c, n - 1) * ld;
-  for (int d = g; d < dh; d += 4) t = __builtin_amdgcn_mfma_f32_16x16x4f32(xr[d], own[d], t, 0, 0, 0);
-  return t;
-}
+// fp32 forms of blocks32 and rows32 from global memory (non-finite values, see gemm_bf3.h), for
+// 16 N rows at a time; the caller issues a step's loads before it uses any.  With one NaN among
+// 16 x 256 x 8 x 64 the forward takes 24 -> 79 us and the backward 48 -> 180 (134 and 310 with
+// 16 rows at a time and each column's load before its MFMA).
 template <class C>
-__device__ __forceinline__ void rows16_fp32(f4 (&acc)[C::NB], const float *x, int64_t ld, int r0, int n,
-                                            f4 p, int dh, int c, int g) {
+struct Fp32 {
+  static constexpr int N = C::DH <= 64 ? 2 : 1, ROWS = 16 * N;
+  float own[C::NB][4];  // the wave's row: columns 16 b + 4 g + j
+  __device__ __forceinline__ void set(const float *row, int dh, int g) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int r = r0 + 4 * g + e;
-    const float *xr = x + (int64_t)min(r, n - 1) * ld;
-#pragma unroll
-    for (int b = 0; b < C::NB; ++b) {
-      const int d = 16 * b + c;
-      const float v = r < n && d < dh ? xr[d] : 0.0f;
-      acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, p[e], acc[b], 0, 0, 0);
-    }
+    for (int b = 0; b < C::NB; ++b) load(own[b], row, 16 * b + 4 * g, dh);
   }
-}
+  static __device__ __forceinline__ void load(float (&v)[4], const float *row, int at, int dh) {
+    const bool in = at < dh;  // dh is a multiple of 8
+    const f4u a = *reinterpret_cast<const f4u *>(row + (in ? at : 0));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = in ? a[j] : 0.0f;
+  }
+  // Rows r0 + 16 u + c of n of `x`, columns 16 b + 4 g + j (past the last: the last row).
+  struct Rows {
+    float v[N][C::NB][4];
+    __device__ __forceinline__ void load(const float *x, int64_t ld, int r0, int n, int dh, int c, int g) {
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int b = 0; b < C::NB; ++b)
+          Fp32::load(v[u][b], x + (int64_t)min(r0 + 16 * u + c, n - 1) * ld, 16 * b + 4 * g, dh);
+    }
+  };
+  // Rows r0 + 16 u + 4 g + e of n of `x`, columns 16 b + c; zero past the last.
+  struct Cols {
+    float v[N][4][C::NB];
+    __device__ __forceinline__ void load(const float *x, int64_t ld, int r0, int n, int dh, int c, int g) {
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = r0 + 16 * u + 4 * g + e;
+          const float *xr = x + (int64_t)min(r, n - 1) * ld;
+#pragma unroll
+          for (int b = 0; b < C::NB; ++b) {
+            const int d = 16 * b + c;
+            const float w = xr[d < dh ? d : 0];
+            v[u][e][b] = r < n && d < dh ? w : 0.0f;
+          }
+        }
+    }
+  };
+  // y[u]: rows r0 + 16 u + 4 g + e against the wave's row.
+  __device__ __forceinline__ void dots(f4 (&y)[N], const Rows &x) const {
+#pragma unroll
+    for (int u = 0; u < N; ++u) y[u] = f4{};
+#pragma unroll
+    for (int b = 0; b < C::NB; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+          y[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[u][b][j], own[b][j], y[u], 0, 0, 0);
+  }
+  // acc[b] += columns 16 b + 4 g + e of the rows times the wave's values p.
+  static __device__ __forceinline__ void add(f4 (&acc)[C::NB], const Cols &x, const f4 (&p)[N]) {
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int b = 0; b < C::NB; ++b)
+          acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[u][e][b], p[u][e], acc[b], 0, 0, 0);
+  }
+};
 
 // The workgroup's head z and first row: XCD k (hardware ids k, k + 8, ...) owns a contiguous
 // run of heads, whose workgroups stage the same rows through one L2.
@@ -533,25 +580,37 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(const float *q, const float 
   join_groups<C>(acc, lds, wave, lane);
   if (grp > 0) return;
   if (any_bad(acc, live)) {  // again in fp32, from global memory
+    using F = Fp32<C>;
+    F f;
+    f.set(q, dh, g);
     st = RowStat{};
-    for (int r0 = 0; r0 < S; r0 += 16) {
-      const f4 y[1] = {block16_fp32(k, ld, r0, S, q, dh, c, g)};
+    for (int r0 = 0; r0 < S; r0 += F::ROWS) {
+      typename F::Rows kr;
+      kr.load(k, ld, r0, S, dh, c, g);
+      f4 y[F::N];
+      f.dots(y, kr);
       st.add<true, false>(y, sc, r0 + 4 * g, S);
     }
     st.join();
     inv = 1.0f / st.l;
 #pragma unroll
     for (int b = 0; b < C::NB; ++b) acc[b] = f4{};
-    for (int r0 = 0; r0 < S; r0 += 16) {
-      const f4 y = block16_fp32(k, ld, r0, S, q, dh, c, g);
-      f4 p;
+    for (int r0 = 0; r0 < S; r0 += F::ROWS) {
+      typename F::Rows kr;
+      typename F::Cols vr;
+      kr.load(k, ld, r0, S, dh, c, g);
+      vr.load(v, ld, r0, S, dh, c, g);
+      f4 y[F::N], p[F::N];
+      f.dots(y, kr);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int key = r0 + 4 * g + e;
-        p[e] = key < S ? __builtin_amdgcn_exp2f(sc.at<true>(y[e], st.m)) * inv : 0.0f;
-        if (live && key < S) Pr[key] = p[e];
-      }
-      rows16_fp32<C>(acc, v, ld, r0, S, p, dh, c, g);
+      for (int u = 0; u < F::N; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = r0 + 16 * u + 4 * g + e;
+          p[u][e] = key < S ? __builtin_amdgcn_exp2f(sc.at<true>(y[u][e], st.m)) * inv : 0.0f;
+          if (live && key < S) Pr[key] = p[u][e];
+        }
+      F::add(acc, vr, p);
     }
   }
   if (live) store_rows<C>(out + ((int64_t)(z / H) * S + row) * ldo + (z % H) * dh, acc, 1.0f, dh, g, 0);
@@ -634,12 +693,22 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
 #pragma unroll
     for (int n = 1; n < C::NG; ++n) d += total[n * 16 * C::NW + r];
     if (__any(live && !(d * 0.0f == 0.0f))) {  // not finite: again in fp32
+      using F = Fp32<C>;
+      F f;
+      f.set(dout + ato, dh, g);
       d = 0.0f;
-      for (int r0 = 0; r0 < S; r0 += 16) {
-        const f4 dp = block16_fp32(v, ld, r0, S, dout + ato, dh, c, g), q = load4(Pr, r0 + 4 * g, S, false);
+      for (int r0 = 0; r0 < S; r0 += F::ROWS) {
+        typename F::Rows vr;
+        vr.load(v, ld, r0, S, dh, c, g);
+        f4 dp[F::N];
+        f.dots(dp, vr);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (r0 + 4 * g + e < S) d += q[e] * dp[e];
+        for (int u = 0; u < F::N; ++u) {
+          const f4 q = load4(Pr, r0 + 16 * u + 4 * g, S, false);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (r0 + 16 * u + 4 * g + e < S) d += q[e] * dp[u][e];
+        }
       }
       d = rows4(d, [](float a, float b) { return a + b; });
     }
@@ -680,12 +749,24 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
   if (any_bad(acc, live)) {
 #pragma unroll
     for (int b = 0; b < C::NB; ++b) acc[b] = f4{};
-    for (int r0 = 0; r0 < S; r0 += 16) {
-      const f4 dp = block16_fp32(v, ld, r0, S, dout + ato, dh, c, g), p = load4(Pr, r0 + 4 * g, S, false);
-      f4 ds;
+    using F = Fp32<C>;
+    F f;
+    f.set(dout + ato, dh, g);
+    for (int r0 = 0; r0 < S; r0 += F::ROWS) {
+      typename F::Rows vr;
+      typename F::Cols kr;
+      vr.load(v, ld, r0, S, dh, c, g);
+      kr.load(k, ld, r0, S, dh, c, g);
+      f4 dp[F::N], ds[F::N];
+      f.dots(dp, vr);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ds[e] = r0 + 4 * g + e < S ? p[e] * (dp[e] - d) : 0.0f;
-      rows16_fp32<C>(acc, k, ld, r0, S, ds, dh, c, g);
+      for (int u = 0; u < F::N; ++u) {
+        const int at = r0 + 16 * u + 4 * g;
+        const f4 p = load4(Pr, at, S, false);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ds[u][e] = at + e < S ? p[e] * (dp[u][e] - d) : 0.0f;
+      }
+      F::add(acc, kr, ds);
     }
   }
   if (live) store_rows<C>(dq + at + (int64_t)row * ld, acc, alpha, dh, g, add);
@@ -786,14 +867,27 @@ __global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const fl
   if (any_bad(av, live) || any_bad(ak, live)) {
 #pragma unroll
     for (int b = 0; b < C::NB; ++b) av[b] = ak[b] = f4{};
-    for (int r0 = 0; r0 < S; r0 += 16) {
-      const f4 dp = block16_fp32(dout, ldo, r0, S, vr, dh, c, g), p = load_p(r0 + 4 * g, false);
-      const f4 d = load4(D, r0 + 4 * g, S, false);
-      f4 ds;
+    using F = Fp32<C>;
+    F f;
+    f.set(vr, dh, g);
+    for (int r0 = 0; r0 < S; r0 += F::ROWS) {
+      typename F::Rows rows;
+      typename F::Cols ocols, qcols;
+      rows.load(dout, ldo, r0, S, dh, c, g);
+      ocols.load(dout, ldo, r0, S, dh, c, g);
+      qcols.load(q, ld, r0, S, dh, c, g);
+      f4 dp[F::N], p[F::N], ds[F::N];
+      f.dots(dp, rows);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ds[e] = r0 + 4 * g + e < S ? p[e] * (dp[e] - d[e]) : 0.0f;
-      rows16_fp32<C>(av, dout, ldo, r0, S, p, dh, c, g);
-      rows16_fp32<C>(ak, q, ld, r0, S, ds, dh, c, g);
+      for (int u = 0; u < F::N; ++u) {
+        const int at = r0 + 16 * u + 4 * g;
+        p[u] = load_p(at, false);
+        const f4 d = load4(D, at, S, false);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ds[u][e] = at + e < S ? p[u][e] * (dp[u][e] - d[e]) : 0.0f;
+      }
+      F::add(av, ocols, p);
+      F::add(ak, qcols, ds);
     }
   }
   if (live) {

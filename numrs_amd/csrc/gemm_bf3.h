@@ -25,7 +25,11 @@
 // Special values.  An infinity, a NaN or a magnitude of 2^112 or more has a term x - h that
 // is not finite, and makes every output of its row or column NaN or infinite; so does a sum
 // of 32 products of 2^96 or more its output.  A wave that finds such an output recomputes
-// its block with fp32 MFMAs, so that the results are those of fp32 arithmetic.
+// its rows or columns of blocks with fp32 MFMAs, so that the results are those of fp32
+// arithmetic.  One such value costs one load's latency per 32 reduction steps: 2048^3 A B^T
+// 109 -> 134 us (the fp32 MFMA kernel: 131), its gradient pair with one NaN in dC 167 -> 293
+// (242), 4096 x 512 -> 2048 forward 64 (66) and backward 178 (135); with four loads in flight
+// in place of forty they took 425, 1205, 220 and 485.
 #pragma once
 
 #include <type_traits>
@@ -356,46 +360,107 @@ struct Product {
     if (__any(bad)) fp32(X, ldx, rows_x, Y, ldy, rows_y, R);
   }
 
-  // The wave's block again with fp32 MFMAs straight from global memory (see "Special
+  // The rows of the wave's 16 x 16 blocks that hold an output that is not finite, or the columns
+  // where those are fewer, again with fp32 MFMAs straight from global memory (see "Special
   // values"): v_mfma_f32_16x16x4f32, lane (g, c) feeding row or column c at reduction step
-  // 4 s + g; sums of 64 steps added into the totals.
+  // 16 s + 4 g + j to MFMA j of 16 steps; sums of 32 steps, whose loads are all issued before the
+  // first MFMA, added into the totals.  Few waves do this, so that a load's latency per 32 steps
+  // and line of blocks is what it costs.  A line at a time keeps it within the product's registers.
   __device__ __forceinline__ void fp32(const float *X, int64_t ldx, int rows_x, const float *Y,
                                        int64_t ldy, int rows_y, int R) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = lane & 15, g = lane >> 4;
-    const int pr = (wave / S::WQ) * (16 * BI) + c, qr = (wave % S::WQ) * (16 * BJ) + c;
-    f4 acc[BI][BJ];
+    using Off = typename std::conditional<S::WIDE, int64_t, uint32_t>::type;
+    unsigned rows = 0, cols = 0;
 #pragma unroll
     for (int i = 0; i < BI; ++i)
 #pragma unroll
-      for (int j = 0; j < BJ; ++j) tot[i][j] = acc[i][j] = f4{};
-    for (int r0 = 0; r0 < R; r0 += 4) {
-      const int64_t r = min(r0 + g, R - 1);
-      const bool in = r0 + g < R;
-      float xv[BI], yv[BJ];
-#pragma unroll
-      for (int i = 0; i < BI; ++i) {
-        const int64_t p = min(pr + 16 * i, rows_x - 1);
-        const float x = XRC ? X[p * ldx + r] : X[r * ldx + p];
-        xv[i] = in ? x : 0.0f;
-      }
-#pragma unroll
       for (int j = 0; j < BJ; ++j) {
-        const int64_t q = min(qr + 16 * j, rows_y - 1);
-        const float y = YRC ? Y[q * ldy + r] : Y[r * ldy + q];
-        yv[j] = in ? y : 0.0f;
+        const f4 z = tot[i][j] * 0.0f;
+        if (__any(!((z[0] + z[1]) + (z[2] + z[3]) == 0.0f))) rows |= 1u << i, cols |= 1u << j;
       }
-      const bool last = r0 + 4 >= R || (r0 & 63) == 60;
+    // Steps k + 4 g .. + 3 of the row whose step 0 is at element `off`.
+    auto load = [&](auto rc, float (&v)[4], const float *base, int64_t ld, Off off, int g, int k) {
+      if constexpr (decltype(rc)::value) {
+        const f4u a = *reinterpret_cast<const f4u *>(base + k + (off + (Off)(4 * g)));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = a[j];
+      } else {
+        const Off at = off + (Off)(4 * g) * (Off)ld;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = (base + (k + j) * ld)[at];
+      }
+    };
+    // Line l of blocks: row l of X's against all of Y's, or column l of Y's against all of X's.
+    auto line = [&](auto row_t, int l, auto &&tot_of) {
+      constexpr bool ROW = decltype(row_t)::value;
+      constexpr int N = ROW ? BJ : BI;
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));  // lane values are not kept from the product or the last line
+      const int lane = tid & 63, wave = tid >> 6;
+      const int c = lane & 15, g = lane >> 4;
+      auto off_x = [&](int b) {
+        const Off r = (Off)min((wave / S::WQ) * (16 * BI) + 16 * b + c, rows_x - 1);
+        return XRC ? r * (Off)ldx : r;
+      };
+      auto off_y = [&](int b) {
+        const Off r = (Off)min((wave % S::WQ) * (16 * BJ) + 16 * b + c, rows_y - 1);
+        return YRC ? r * (Off)ldy : r;
+      };
+      const Off off = ROW ? off_x(l) : off_y(l);
+      using One = std::integral_constant<bool, ROW ? XRC : YRC>;
+      using All = std::integral_constant<bool, ROW ? YRC : XRC>;
+      const float *const A = ROW ? X : Y, *const B = ROW ? Y : X;
+      const int64_t lda = ROW ? ldx : ldy, ldb = ROW ? ldy : ldx;
+      auto mfma = [&](float one, float other, f4 t) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(ROW ? one : other, ROW ? other : one, t, 0, 0, 0);
+      };
+      Off all[N];
+      f4 t[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        all[n] = ROW ? off_y(n) : off_x(n);
+        tot_of(n) = t[n] = f4{};
+      }
+      int r0 = 0;
+#pragma unroll 1
+      for (; r0 + 32 <= R; r0 += 32) {
+        float a[2][4], b[2][N][4];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          load(One{}, a[u], A, lda, off, g, r0 + 16 * u);
+#pragma unroll
+          for (int n = 0; n < N; ++n) load(All{}, b[u][n], B, ldb, all[n], g, r0 + 16 * u);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int n = 0; n < N; ++n) t[n] = mfma(a[u][e], b[u][n][e], t[n]);
+#pragma unroll
+        for (int n = 0; n < N; ++n) tot_of(n) += t[n], t[n] = f4{};
+      }
+#pragma unroll 1
+      for (; r0 < R; r0 += 4) {  // fewer than 32 steps: step r0 + g
+        const bool in = r0 + g < R;
+        const int64_t r = in ? r0 + g : 0;
+        const float a = A[(int64_t)off + (One::value ? r : r * lda)];
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+          const float b = B[(int64_t)all[n] + (All::value ? r : r * ldb)];
+          t[n] = mfma(in ? a : 0.0f, in ? b : 0.0f, t[n]);
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < N; ++n) tot_of(n) += t[n];
+    };
+    if (__builtin_popcount(rows) <= __builtin_popcount(cols)) {
 #pragma unroll
       for (int i = 0; i < BI; ++i)
+        if (rows >> i & 1) line(std::true_type{}, i, [&](int n) -> f4 & { return tot[i][n]; });
+    } else {
 #pragma unroll
-        for (int j = 0; j < BJ; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[i], yv[j], acc[i][j], 0, 0, 0);
-          if (last) {
-            tot[i][j] += acc[i][j];
-            acc[i][j] = f4{};
-          }
-        }
+      for (int j = 0; j < BJ; ++j)
+        if (cols >> j & 1) line(std::false_type{}, j, [&](int n) -> f4 & { return tot[n][j]; });
     }
   }
 };

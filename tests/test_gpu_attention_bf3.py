@@ -173,3 +173,55 @@ def test_small_values(hip_ctx, B, S, H, dh, given):
             dS = p * (dP - (dP * p).sum(-1, keepdims=True)) / math.sqrt(dh)
             # dP - D cancels: errors of 5e-7 of dP's size, not of the difference's
             assert rel(split(dk.numpy())[:, 1:], (dS.transpose(0, 1, 3, 2) @ Q)[:, 1:]) < 4e-6
+
+
+def _same_kind(got, ref, what):
+    """NaN and infinities where the reference has them, the rest within fp32's rounding of the
+    head's largest value ([.., S, dh] arrays)."""
+    assert np.array_equal(np.isnan(got), np.isnan(ref)), f"{what}: NaN"
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)]), f"{what}: inf"
+    fine = np.isfinite(ref)
+    top = np.abs(np.where(fine, ref, 0.0)).max(axis=(-2, -1), keepdims=True)
+    err = np.abs(np.where(fine, got - np.where(fine, ref, 0.0), 0.0))
+    assert np.all(err <= 2e-5 * top), f"{what}: {(err / np.maximum(top, 1e-300)).max()}"
+
+
+# eight row groups of 16 and four, heads of 8 to 128
+@pytest.mark.parametrize("B,S,H,dh", [(16, 200, 16, 64), (2, 300, 16, 64), (2, 200, 12, 32), (8, 257, 12, 72),
+                                      (3, 520, 30, 128)])
+@pytest.mark.parametrize("given", [True, False])
+def test_backward_special_values(hip_ctx, B, S, H, dh, given):
+    """Infinities, NaN and magnitudes of 2^112 and more in Q, K, V and dO: the gradients that
+    fp32 arithmetic gives (float64 here, of the GPU's own P and output)."""
+    print(f"[gpu] attention special values B={B} S={S} H={H} dh={dh} out={given}", flush=True)
+    rng = np.random.default_rng(9)
+    D, c, lib = H * dh, hip_ctx, L.load()
+    q, k, v, g = (rand(rng, (B * S, D)) for _ in range(4))
+    g[5, 3] = np.inf                        # head 0
+    v[7, dh + 1] = np.inf                   # head 1
+    q[9, 2 * dh + 2] = np.inf               # head 2
+    g[11, 3 * dh], v[:S, 3 * dh] = 3.395e38, 1e-3 * v[:S, 3 * dh]
+    k[20, 4 * dh + 2], q[:S, 4 * dh + 2] = 1e36, 0.0
+    g[S - 1, 5 * dh + 4] = np.nan
+    qd, kd, vd, gd = (c.to_device(a) for a in (q, k, v, g))
+    P, out, dq, dk, dv = c.empty((B * H, S, S)), *(c.empty((B * S, D)) for _ in range(4))
+    assert lib.numrs_hip_attention_forward(c.handle, qd.ptr, kd.ptr, vd.ptr, P.ptr, out.ptr, B, S, H, D) == 0
+    if given:
+        rc = lib.numrs_hip_attention_backward_out_strided(
+            c.handle, qd.ptr, kd.ptr, vd.ptr, D, P.ptr, out.ptr, gd.ptr, D, dq.ptr, dk.ptr, dv.ptr, B, S, H, D, 0)
+    else:
+        rc = lib.numrs_hip_attention_backward(c.handle, qd.ptr, kd.ptr, vd.ptr, P.ptr, gd.ptr, dq.ptr, dk.ptr,
+                                              dv.ptr, B, S, H, D, 0)
+    assert rc == 0
+    split = lambda a: a.astype(np.float64).reshape(B, S, H, dh).transpose(0, 2, 1, 3)  # noqa: E731
+    Q, K, V, G, O = (split(a) for a in (q, k, v, g, out.numpy()))
+    p = P.numpy().astype(np.float64).reshape(B, H, S, S)
+    with np.errstate(all="ignore"):
+        dP = G @ V.transpose(0, 1, 3, 2)
+        total = (G * O).sum(-1, keepdims=True) if given else (p * dP).sum(-1, keepdims=True)
+        dS = p * (dP - total)
+        alpha = 1 / math.sqrt(dh)
+        dK, dQ, dV = alpha * (dS.transpose(0, 1, 3, 2) @ Q), alpha * (dS @ K), p.transpose(0, 1, 3, 2) @ G
+    _same_kind(split(dv.numpy()), dV, "dv")
+    _same_kind(split(dq.numpy()), dQ, "dq")
+    _same_kind(split(dk.numpy()), dK, "dk")

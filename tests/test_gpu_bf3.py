@@ -137,6 +137,30 @@ def test_special_values(hip_ctx, rng, ta, tb):
     assert tiny.max() <= 1e-6 * np.sqrt(K) * 1e-30
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,K,N", SIZES)
+def test_special_values_of_every_shape(hip_ctx, rng, M, K, N, ta, tb):
+    """A row, a column and their crossing that hold an infinity, a NaN or a value above 2^112,
+    in the first and last blocks of every tile shape; every other output as without them."""
+    print(f"[gpu] bf3 special values {M}x{K}x{N} ta={ta} tb={tb}", flush=True)
+    A, B = rand(rng, (M, K)), rand(rng, (K, N))
+    A[0, K - 1], A[M - 1, 0], A[M // 2, K // 2] = np.inf, 1e35, np.nan
+    B[K // 3, N - 1], B[K - 1, 1] = -np.inf, 1e35
+    got = _product(hip_ctx, np.ascontiguousarray(A.T) if ta else A,
+                   np.ascontiguousarray(B.T) if tb else B, ta, tb)
+    with np.errstate(all="ignore"):
+        ref = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fine = np.isfinite(ref)
+    large = np.zeros(ref.shape, bool)
+    large[M - 1], large[:, 1] = True, True
+    assert_contraction(got[fine & ~large], ref[fine & ~large], K, what="others")
+    # sums of at most a few terms above the rest: rounded at their size
+    rest = fine & large
+    assert np.all(np.abs(got[rest] - ref[rest]) <= 1e-6 * np.abs(ref[rest]) + 1e-6 * 1e35)
+
+
 @pytest.mark.parametrize("K", [64, 512, 2048])
 def test_mean_error(hip_ctx, rng, K):
     """The matrix unit's sums round down; tiles of alternating sign cancel that.  Without them
