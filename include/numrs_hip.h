@@ -332,12 +332,12 @@ int numrs_hip_attention_backward_strided(numrs_hip_ctx *ctx, const float *q, con
                                          float *dv, int64_t B, int64_t S, int64_t H, int64_t D,
                                          int accumulate);
 /* The backward given also the forward's output out (rows at ld_out, like
- * dout), from which the softmax backward's row totals come as dO . O.  Larger
- * calls (D/H a multiple of 8 up to 128) run two kernels in both forms: one
- * over query rows (the row totals, into B*H*S floats of the context's memory,
- * and dQ), then one over key rows (dV and dK); without out the first walks
- * the keys once more.  Every output element is written once, with no
- * atomics. */
+ * dout), from which the softmax backward's row totals come as dO . O.  Most
+ * calls with D/H a multiple of 8 up to 128 run a kernel over query rows (the
+ * row totals, into B*H*S floats of the context's memory, and dQ) and one over
+ * key rows (dV and dK), small ones both in one launch; without out the first
+ * walks the keys once more.  Every output element is written once, with no
+ * atomics.  The grads must not overlap any input. */
 int numrs_hip_attention_backward_out_strided(numrs_hip_ctx *ctx, const float *q, const float *k,
                                              const float *v, int64_t ld_qkv, const float *P,
                                              const float *out, const float *dout, int64_t ld_out,

@@ -25,18 +25,38 @@ bool fills(numrs_hip_ctx *ctx, int64_t S, int64_t Z) {
   return (S + 127) / 128 * Z * 4 >= 3 * std::max(ctx->num_cus, 1);
 }
 
-// attention_bf3.h's kernels: head sizes of whole 16-byte chunks up to 128; a staged block
-// and four rows of P within 31-bit element offsets.  Below 2^24 multiply-adds a product
-// (the tiny GEMM's range), with fewer than 32 workgroups, or with heads above 64 on a part of
-// the chip, the GEMMs and row kernels are as fast or faster.  Forward and backward on MI355X,
-// B x S x H x dh, kernels | GEMMs: 4 x 128 x 4 x 64 28 | 40 us, 2 x 256 x 4 x 64 43 | 57, 16 x 64 x
-// 16 x 128 46 | 55, 1 x 1000 x 4 x 64 143 | 157; 4 x 64 x 4 x 64 30 | 24, 1 x 1000 x 1 x 64 140 | 73,
-// 4 x 256 x 8 x 128 92 | 76.
-bool bf3_fits(numrs_hip_ctx *ctx, int64_t B, int64_t S, int64_t H, int64_t dh, int64_t li, int64_t lo) {
-  const int64_t Z = B * H;
+// Whether attention_bf3.h's kernels take the call: head sizes of whole 16-byte chunks up to 128; a
+// staged block and four rows of P within 31-bit element offsets.
+bool bf3_takes(int64_t S, int64_t Z, int64_t dh, int64_t li, int64_t lo) {
   return dh % 8 == 0 && dh <= 128 && Z < 65536 && S < (int64_t{1} << 28) && li < (int64_t{1} << 24) &&
-         lo < (int64_t{1} << 24) && (double)Z * S * S * dh >= (double)(1 << 24) && (S + 63) / 64 * Z >= 32 &&
-         (dh <= 64 || fills(ctx, S, Z));
+         lo < (int64_t{1} << 24);
+}
+
+// And whether they are the faster ones.  Below 2^24 multiply-adds a product (the tiny GEMM's
+// range), with fewer than 32 workgroups, or with heads above 64 on a part of the chip, the GEMMs
+// and row kernels are as fast or faster: forward and backward on MI355X, B x S x H x dh,
+// kernels | GEMMs: 2 x 256 x 4 x 64 43 | 57 us, 16 x 64 x 16 x 128 46 | 55, 1 x 1000 x 4 x 64 143 |
+// 157; 1 x 1000 x 1 x 64 140 | 73, 4 x 256 x 8 x 128 92 | 76.
+bool bf3_fits(numrs_hip_ctx *ctx, int64_t S, int64_t Z, int64_t dh, int64_t li, int64_t lo) {
+  return bf3_takes(S, Z, dh, li, lo) && (double)Z * S * S * dh >= (double)(1 << 24) &&
+         (S + 63) / 64 * Z >= 32 && (dh <= 64 || fills(ctx, S, Z));
+}
+
+// Heads up to 64 and at most one staged block of 128 rows, or whole ones up to `most`, a workgroup
+// to a CU: one launch in place of three or six.  Forward, one head of 64 and eight, kernel | GEMMs:
+// S = 64 8 | 10 and 9 | 11 us, 128 8 | 11 and 8 | 13, 256 12 | 14, 384 with four 17 | 26, 512 with
+// two 21 | 30; but 192 13 | 12, 320 17 | 15.  Backward with the output: 64 11 | 13 and 12 | 14, 128
+// 11 | 15 and 11 | 17, 256 17 | 19 and 18 | 30; but 192 17 | 15, 384 23 | 22, 512 29 | 24.
+bool bf3_few(numrs_hip_ctx *ctx, int64_t S, int64_t Z, int64_t dh, int64_t li, int64_t lo, int64_t most) {
+  return bf3_takes(S, Z, dh, li, lo) && dh <= 64 && (S + 63) / 64 * Z <= ctx->num_cus &&
+         (S <= 128 || (S <= most && S % 128 == 0));
+}
+
+// Whether the backward with the output runs as one launch (attn::bwd_both_kernel): its workgroups
+// of both kinds at most one to a CU.  Above that the two launches are as fast or faster: S = 384,
+// 32 heads 42 us against 47, S = 512, 32 heads 55 against 61.
+bool both_fit(numrs_hip_ctx *ctx, int64_t S, int64_t Z, int64_t dh) {
+  return dh <= 64 && S <= attn::kMaxS && (S + 63) / 64 * Z * 2 <= ctx->num_cus && !fills(ctx, S, Z);
 }
 
 // Calls f with the configuration for head size dh and its grid: eight row groups of 16 where
@@ -64,24 +84,41 @@ void with_bf3(numrs_hip_ctx *ctx, int64_t S, int64_t Z, int64_t dh, F &&f) {
   }
 }
 
-// The two backward kernels: D (from `out` where given) and dQ, then dV and dK; any of the three
-// may be null.
+// The backward kernels: D (from `out` where given) and dQ, then dV and dK, or all at once; any of
+// the three may be null.
 int bf3_backward(numrs_hip_ctx *ctx, const float *q, const float *k, const float *v, int64_t li, const float *P,
                  const float *out, const float *dout, int64_t lo, float *dq, float *dk, float *dv, int64_t B,
                  int64_t S, int64_t H, int64_t dh, int accumulate) {
   const float alpha = 1.0f / sqrtf((float)dh);
+  const bool both = dq != nullptr && (dk != nullptr || dv != nullptr) && both_fit(ctx, S, B * H, dh);
   numrs_hip::TempBlock rows(ctx);  // D per query, from the first kernel to the second
-  if (int rc = rows.alloc((size_t)(B * H * S) * sizeof(float))) return rc;
+  if (out == nullptr || !both)
+    if (int rc = rows.alloc((size_t)(B * H * S) * sizeof(float))) return rc;
   float *D = rows.f();
   with_bf3(ctx, S, B * H, dh, [&](auto cfg, dim3 grid) {
     using C = decltype(cfg);
     const int l = (int)li, s = (int)S, h = (int)H, d = (int)dh;
+    auto query = [&](auto mode, float *grad) {
+      attn::bwd_query_kernel<C, decltype(mode)::value><<<grid, C::NT, 0, ctx->stream>>>(
+          k, v, l, P, dout, out, lo, D, grad, s, h, d, alpha, accumulate);
+    };
+    const std::integral_constant<int, attn::kWalkD> walk;
+    const std::integral_constant<int, attn::kOutD> from_out;
+    if constexpr (C::NG > 1) {  // both_fit: only these
+      auto together = [&](auto given) {
+        attn::bwd_both_kernel<C, decltype(given)::value><<<dim3(2 * grid.x, grid.y), C::NT, 0, ctx->stream>>>(
+            q, k, v, l, P, dout, out, (int)lo, D, dq, dk, dv, s, h, d, alpha, accumulate);
+      };
+      if (both && out != nullptr) return together(std::true_type{});
+      if (both) {
+        query(walk, nullptr);
+        return together(std::false_type{});
+      }
+    }
     if (out != nullptr)
-      attn::bwd_query_kernel<C, true><<<grid, C::NT, 0, ctx->stream>>>(k, v, l, P, dout, out, lo, D, dq, s, h, d,
-                                                                       alpha, accumulate);
+      query(from_out, dq);
     else
-      attn::bwd_query_kernel<C, false><<<grid, C::NT, 0, ctx->stream>>>(k, v, l, P, dout, out, lo, D, dq, s, h, d,
-                                                                        alpha, accumulate);
+      query(walk, dq);
     if (dk != nullptr || dv != nullptr)
       attn::bwd_key_kernel<C><<<grid, C::NT, 0, ctx->stream>>>(q, v, l, P, dout, (int)lo, D, dk, dv, s, h, d, alpha,
                                                                accumulate);
@@ -116,18 +153,21 @@ int numrs_hip_attention_forward_strided(numrs_hip_ctx *ctx, const float *q, cons
     return numrs_hip::fail(ctx, NUMRS_HIP_E_INVALID, "attention_forward: null pointer");
   const int64_t dh = D / H, Z = B * H, li = ld_qkv, lo = ld_out;
   const float alpha = 1.0f / sqrtf((float)dh);
-  if (bf3_fits(ctx, B, S, H, dh, li, lo)) {
+  if (bf3_fits(ctx, S, Z, dh, li, lo) || bf3_few(ctx, S, Z, dh, li, lo, 512)) {
     const double a2 = (double)alpha * 1.4426950408889634;  // alpha log2 e
     const attn::Scale sc{(float)a2, (float)(a2 - (double)(float)a2)};
     with_bf3(ctx, S, Z, dh, [&](auto cfg, dim3 grid) {
       using C = decltype(cfg);
-      constexpr int kKeep = 256 / C::BLK;  // all scores of a wave in registers
-      if (S <= 256)
-        attn::fwd_kernel<C, kKeep><<<grid, C::NT, 0, ctx->stream>>>(q, k, v, (int)li, P, out, lo, (int)S, (int)H,
-                                                                    (int)dh, sc);
-      else
-        attn::fwd_kernel<C, 0><<<grid, C::NT, 0, ctx->stream>>>(q, k, v, (int)li, P, out, lo, (int)S, (int)H,
-                                                                (int)dh, sc);
+      auto go = [&](auto keep) {
+        attn::fwd_kernel<C, decltype(keep)::value><<<grid, C::NT, 0, ctx->stream>>>(
+            q, k, v, (int)li, P, out, lo, (int)S, (int)H, (int)dh, sc);
+      };
+      // all scores of a wave in registers: those of 256 keys, with the keys of a block halved
+      // between two sets of waves of 512
+      if (S <= 256) return go(std::integral_constant<int, 256 / C::BLK>{});
+      if constexpr (C::NG > 1)
+        if (S <= 512) return go(std::integral_constant<int, 512 / C::BLK>{});
+      go(std::integral_constant<int, 0>{});
     });
     return numrs_hip::check_launch(ctx, "attn::fwd_kernel");
   }
@@ -159,7 +199,7 @@ int numrs_hip_attention_backward_strided(numrs_hip_ctx *ctx, const float *q, con
                           H * S * S, S * S, S * lo, dh, S * li, dh);
   };
   if (!dq && !dk) return dv ? dv_gemm() : NUMRS_HIP_OK;
-  if (bf3_fits(ctx, B, S, H, dh, li, lo))
+  if (bf3_fits(ctx, S, Z, dh, li, lo))
     return bf3_backward(ctx, q, k, v, li, P, nullptr, dout, lo, dq, dk, dv, B, S, H, dh, accumulate);
   // dS lives in a block of its own: the products below may split their
   // reduction and write partials to the context workspace while reading dS.
@@ -192,7 +232,9 @@ int numrs_hip_attention_backward_out_strided(numrs_hip_ctx *ctx, const float *q,
   if (int rc = check(ctx, B, S, H, D, ld_qkv, ld_out)) return rc;
   if (!q || !k || !v || !P || !dout || !out)
     return numrs_hip::fail(ctx, NUMRS_HIP_E_INVALID, "attention_backward: null input");
-  if ((dq || dk) && bf3_fits(ctx, B, S, H, D / H, ld_qkv, ld_out))
+  const int64_t Z = B * H, dh = D / H;
+  if ((dq || dk) && (bf3_fits(ctx, S, Z, dh, ld_qkv, ld_out) ||
+                     (bf3_few(ctx, S, Z, dh, ld_qkv, ld_out, 256) && both_fit(ctx, S, Z, dh) && dq && (dk || dv))))
     return bf3_backward(ctx, q, k, v, ld_qkv, P, out, dout, ld_out, dq, dk, dv, B, S, H, D / H, accumulate);
   return numrs_hip_attention_backward_strided(ctx, q, k, v, ld_qkv, P, dout, ld_out, dq, dk, dv, B, S, H, D,
                                               accumulate);

@@ -4,6 +4,7 @@
 //   forward        P = softmax(alpha Q K^T) stored, O = P V
 //   query rows     D = dO . O, dS = P (dO V^T - D), dQ = alpha dS K
 //   key rows       dV = P^T dO, dK = alpha dS^T Q, with dS formed again from P, dO V^T and D
+// (the two in one launch where they are few)
 //
 // A wave owns 16 rows (of queries, or keys in the last kernel) as the columns c of its MFMAs;
 // the workgroup walks the other sequence in blocks of BLK rows staged in LDS.  The first
@@ -616,19 +617,17 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(const float *q, const float 
   if (live) store_rows<C>(out + ((int64_t)(z / H) * S + row) * ldo + (z % H) * dh, acc, 1.0f, dh, g, 0);
 }
 
-// D[z, row], the softmax backward's row total of P dP, and dQ (null: D alone).  OUT: from the
-// forward's output, D = dO . (P V) = dO . O; otherwise a walk over the keys of its own.
-template <class C, bool OUT>
-__global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const float *v, int ld,
-                                                          const float *P, const float *dout, const float *out,
-                                                          int64_t ldo, float *D, float *dq, int S, int H, int dh,
-                                                          float alpha, int add) {
-  __shared__ __attribute__((aligned(1024))) char lds[2 * C::kImage];
+// D[z, row], the softmax backward's row total of P dP, and dQ (null: D alone).  D comes from a walk
+// over the keys of its own, from the forward's output, D = dO . (P V) = dO . O, or is given.
+// Workgroup blk of head z; lds: two images.
+enum { kWalkD, kOutD, kGivenD };
+template <class C, int MODE>
+__device__ __forceinline__ void bwd_query(char *lds, int z, int blk, const float *k, const float *v, int ld,
+                                          const float *P, const float *dout, const float *out, int64_t ldo,
+                                          float *D, float *dq, int S, int H, int dh, float alpha, int add) {
   static_assert(C::parts_fit(2), "partial outputs");
   char *const vl = lds, *const kl = lds + C::kImage;
   constexpr int N16 = C::N16;
-  int z, blk;
-  place(z, blk);
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = wave / C::NW, n0 = grp * N16;
   const int row = blk * 16 * C::NW + wave % C::NW * 16 + c;
@@ -657,7 +656,9 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
     for (int n = 0; n < N16; ++n) p[n] = load4(Pr, first(i) + 16 * n + 4 * g, S, first(i) + C::SUB <= S);
   };
   float d = 0.0f;
-  if constexpr (OUT) {
+  if constexpr (MODE == kGivenD) {
+    d = D[(int64_t)z * S + rc];
+  } else if constexpr (MODE == kOutD) {
 #pragma unroll
     for (int s = 0; s < C::NS; ++s)
       if (32 * s + 8 * g < dh)
@@ -669,8 +670,8 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
     walk<0>(
         nb, [&](int i) { vb.load(v, ld, i * C::BLK, S, tid); },
         [&]() {
-          vb.store(vl, tid);
           load_p(next++);
+          vb.store(vl, tid);
         },
         [&](int) {
           float part = 0.0f;
@@ -714,7 +715,7 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
     }
     next = 0;
   }
-  if (live && g == 0 && grp == 0) D[(int64_t)z * S + row] = d;
+  if (MODE != kGivenD && D != nullptr && live && g == 0 && grp == 0) D[(int64_t)z * S + row] = d;
   if (dq == nullptr) return;
   walk<0>(
       nb,
@@ -723,9 +724,9 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
         kb.load(k, ld, i * C::BLK, S, tid);
       },
       [&]() {
+        load_p(next++);
         vb.store(vl, tid);
         kb.store(kl, tid);
-        load_p(next++);
       },
       [&](int i) {
 #pragma unroll
@@ -772,17 +773,14 @@ __global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const 
   if (live) store_rows<C>(dq + at + (int64_t)row * ld, acc, alpha, dh, g, add);
 }
 
-// dV and dK (either may be null), given D.
+// dV and dK (either may be null), given D (of head z).  Workgroup blk of head z; lds: three images.
 template <class C>
-__global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const float *v, int ld, const float *P,
-                                                        const float *dout, int ldo, const float *D, float *dk,
-                                                        float *dv, int S, int H, int dh, float alpha, int add) {
-  __shared__ __attribute__((aligned(1024))) char lds[3 * C::kImage];
+__device__ __forceinline__ void bwd_key(char *lds, int z, int blk, const float *q, const float *v, int ld,
+                                        const float *P, const float *dout, int ldo, const float *D, float *dk,
+                                        float *dv, int S, int H, int dh, float alpha, int add) {
   static_assert(C::parts_fit(3), "partial outputs");
   char *const ol = lds, *const otl = lds + C::kImage, *const ql = lds + 2 * C::kImage;
   constexpr int N16 = C::N16;
-  int z, blk;
-  place(z, blk);
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = wave / C::NW, n0 = grp * N16;
   const int row = blk * 16 * C::NW + wave % C::NW * 16 + c;
@@ -795,7 +793,6 @@ __global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const fl
   Terms own[C::NS];
   own_rows<C>(own, vr, dh, g);
   const float *Pc = P + (int64_t)z * S * S + rc;
-  D += (int64_t)z * S;
   Block<C, false> ob;
   Block<C, true> otb, qb;
   const int nb = (S + C::BLK - 1) / C::BLK;
@@ -829,9 +826,6 @@ __global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const fl
         qb.load(q, ld, i * C::BLK, S, tid);
       },
       [&]() {
-        ob.store(ol, tid);
-        otb.store(otl, tid);
-        qb.store(ql, tid);
         const int r0 = first(next++);
         const bool whole = r0 + C::SUB <= S;
 #pragma unroll
@@ -839,6 +833,9 @@ __global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const fl
           p[n] = load_p(r0 + 16 * n + 4 * g, whole);
           d[n] = load4(D, r0 + 16 * n + 4 * g, S, whole);
         }
+        ob.store(ol, tid);
+        otb.store(otl, tid);
+        qb.store(ql, tid);
       },
       [&](int i) {
 #pragma unroll
@@ -893,6 +890,76 @@ __global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const fl
   if (live) {
     if (dv != nullptr) store_rows<C>(dv + at + (int64_t)row * ld, av, 1.0f, dh, g, add);
     if (dk != nullptr) store_rows<C>(dk + at + (int64_t)row * ld, ak, alpha, dh, g, add);
+  }
+}
+
+template <class C, int MODE>
+__global__ void __launch_bounds__(C::NT) bwd_query_kernel(const float *k, const float *v, int ld, const float *P,
+                                                          const float *dout, const float *out, int64_t ldo,
+                                                          float *D, float *dq, int S, int H, int dh, float alpha,
+                                                          int add) {
+  __shared__ __attribute__((aligned(1024))) char lds[2 * C::kImage];
+  int z, blk;
+  place(z, blk);
+  bwd_query<C, MODE>(lds, z, blk, k, v, ld, P, dout, out, ldo, D, dq, S, H, dh, alpha, add);
+}
+
+template <class C>
+__global__ void __launch_bounds__(C::NT) bwd_key_kernel(const float *q, const float *v, int ld, const float *P,
+                                                        const float *dout, int ldo, const float *D, float *dk,
+                                                        float *dv, int S, int H, int dh, float alpha, int add) {
+  __shared__ __attribute__((aligned(1024))) char lds[3 * C::kImage];
+  int z, blk;
+  place(z, blk);
+  bwd_key<C>(lds, z, blk, q, v, ld, P, dout, ldo, D + (int64_t)z * S, dk, dv, S, H, dh, alpha, add);
+}
+
+// Both at once, for heads of at most 64 and S <= kMaxS: 2 x nx workgroups a head.  With the
+// forward's output the key ones form the head's D = dO . O themselves; else D is given.  A
+// workgroup's chain of loads, splits and MFMAs bounds either kind, so that where one launch leaves
+// CUs idle the two together take little longer than one: with the output 64 x 128 x 64 (heads x S x
+// dh) 20 -> 12 us, 16 x 256 x 64 30 -> 18, 8 x 512 x 64 49 -> 30; without, D's own launch
+// included, 64 x 128 x 64
+// 21 -> 17, 32 x 256 x 64 33 -> 25, 16 x 512 x 64 56 -> 41.
+constexpr int kMaxS = 512;
+template <class C, bool OUT>
+__global__ void __launch_bounds__(C::NT) bwd_both_kernel(const float *q, const float *k, const float *v, int ld,
+                                                         const float *P, const float *dout, const float *out,
+                                                         int ldo, float *D, float *dq, float *dk, float *dv, int S,
+                                                         int H, int dh, float alpha, int add) {
+  static_assert(C::DH <= 64 && C::NT % 8 == 0, "eight lanes a row");
+  __shared__ __attribute__((aligned(1024))) char lds[3 * C::kImage];
+  int z, blk;
+  place(z, blk);
+  const int nx = gridDim.x / 2;
+  if (blk < nx) {
+    bwd_query<C, OUT ? kOutD : kGivenD>(lds, z, blk, k, v, ld, P, dout, out, ldo, OUT ? nullptr : D, dq, S, H, dh,
+                                        alpha, add);
+  } else if constexpr (!OUT) {
+    bwd_key<C>(lds, z, blk - nx, q, v, ld, P, dout, ldo, D + (int64_t)z * S, dk, dv, S, H, dh, alpha, add);
+  } else {
+    __shared__ __attribute__((aligned(16))) float Dz[kMaxS];
+    const int64_t at = (int64_t)(z / H) * S * ldo + (z % H) * dh;
+    const int col = threadIdx.x % 8 * 8;
+#pragma unroll 2
+    for (int r0 = 0; r0 < S; r0 += C::NT / 8) {
+      const int r = r0 + threadIdx.x / 8;
+      const int64_t from = at + (int64_t)min(r, S - 1) * ldo + (col < dh ? col : 0);
+      float d = 0.0f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const f4u a = *reinterpret_cast<const f4u *>(dout + from + 4 * h);
+        const f4u b = *reinterpret_cast<const f4u *>(out + from + 4 * h);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d += a[j] * b[j];
+      }
+      if (col >= dh) d = 0.0f;
+#pragma unroll
+      for (int m = 1; m < 8; m *= 2) d += __shfl_xor(d, m);
+      if (r < S && col == 0) Dz[r] = d;
+    }
+    // the first barrier of bwd_key's walk stands before any read of Dz
+    bwd_key<C>(lds, z, blk - nx, q, v, ld, P, dout, ldo, Dz, dk, dv, S, H, dh, alpha, add);
   }
 }
 

@@ -11,14 +11,21 @@ from numrs_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
 
-# Each above 2^24 multiply-adds per product and 32 workgroups.  Eight row groups (enough
-# workgroups to fill the chip) or four; sequences below and above 256 (scores kept or formed
-# again); heads of 8 (padded to 32), 24, 40 and 64, 72 (to 96), 128 (the last shape, heads of 96 on part
-# of the chip, keeps the GEMMs); sequences one past, one
-# short of and far from a block's end; 16 x 256 x 8 x 64 is the encoder block's.
+# Eight row groups (enough workgroups to fill the chip) or four; sequences below and above 256
+# (scores kept or formed again; four row groups: 512); heads of 8 (padded to 32), 24, 40 and 64, 72
+# (to 96) and 128; sequences one past, one short of and far from a block's end; 16 x 256 x 8 x 64 is
+# the encoder block's.  Both kinds of the backward's workgroups in one launch (without the output
+# after another for D): (2, 300, 16, 32), (2, 511, 8, 64) (on all CUs) and the small ones; a launch
+# each: (2, 300, 24, 32).  Below
+# 2^24 multiply-adds one launch of few workgroups: (1, 1, 1, 8) to (4, 128, 4, 64), and (2, 128, 1,
+# 64), (1, 256, 7, 64), (1, 512, 2, 64; its backward takes the GEMMs); all of them GEMMs: (1, 192, 2,
+# 64), and heads of 96 on part of the chip.  (2, 200, 12, 32) and (8, 250, 20, 128): heads up to 32
+# on part of the chip and of 128 on all of it, with the scores kept.
 SHAPES = [(4, 130, 8, 40), (16, 129, 16, 8), (2, 300, 16, 32), (8, 257, 12, 72), (32, 100, 16, 24),
           (3, 520, 30, 128), (10, 255, 10, 96), (5, 321, 7, 64), (16, 256, 8, 64), (4, 383, 24, 64),
-          (2, 300, 16, 96)]
+          (2, 300, 16, 96), (2, 511, 8, 64), (2, 300, 24, 32), (1, 1, 1, 8), (3, 5, 2, 16), (2, 64, 3, 64),
+          (1, 65, 2, 40), (1, 127, 5, 64), (4, 128, 4, 64), (2, 128, 1, 64), (1, 256, 7, 64), (1, 512, 2, 64),
+          (1, 384, 4, 56), (1, 192, 2, 64), (2, 200, 12, 32), (8, 250, 20, 128)]
 
 
 def _ref(q, k, v, g, B, S, H):
@@ -186,9 +193,10 @@ def _same_kind(got, ref, what):
     assert np.all(err <= 2e-5 * top), f"{what}: {(err / np.maximum(top, 1e-300)).max()}"
 
 
-# eight row groups of 16 and four, heads of 8 to 128
-@pytest.mark.parametrize("B,S,H,dh", [(16, 200, 16, 64), (2, 300, 16, 64), (2, 200, 12, 32), (8, 257, 12, 72),
-                                      (3, 520, 30, 128)])
+# eight row groups of 16 and four (with the output in one launch, but for 2 x 400 x 20), heads of 8
+# to 128
+@pytest.mark.parametrize("B,S,H,dh", [(16, 200, 16, 64), (2, 300, 16, 64), (2, 200, 12, 32), (4, 383, 10, 64),
+                                      (2, 400, 20, 48), (8, 257, 12, 72), (3, 520, 30, 128)])
 @pytest.mark.parametrize("given", [True, False])
 def test_backward_special_values(hip_ctx, B, S, H, dh, given):
     """Infinities, NaN and magnitudes of 2^112 and more in Q, K, V and dO: the gradients that
