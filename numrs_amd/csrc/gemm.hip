@@ -54,8 +54,9 @@ struct Gemm {
   int accumulate;
   float alpha;  // C = alpha * X@Y (+ C)
   // Split-K: with splits > 1 the reduction is cut into `splits` ranges of
-  // whole k-tiles; range s writes its plain partial product to
-  // partial + s*P*Q (row stride Q) and splitk_reduce forms alpha*sum (+C).
+  // whole k-tiles; range s of batch z writes its plain partial product to
+  // partial + (z*splits + s)*P*Q (row stride Q) and splitk_reduce forms
+  // alpha*sum (+C).
   int splits;
   int ktiles_per_split;
   float *partial;
@@ -92,7 +93,8 @@ __device__ __forceinline__ float act_value(int act, float v) {
 }
 
 // One split product's reduction: C = alpha * sum_s partial[s] (+ bias[q])
-// (+ C), partial s at partial + s*n with row stride Q.
+// (+ C), partial s at partial + s*n with row stride Q; batch z (blockIdx.z) at
+// partial + z*splits*n, its C as Gemm's.
 struct SplitSet {
   const float *partial;
   float *C;
@@ -105,6 +107,8 @@ struct SplitSet {
   const float *res;  // residual added after the bias (row stride ldr)
   int64_t ldr;
   int kahan;  // the splits added as a compensated (Kahan) sum, in the same order
+  int64_t bsc, bsc2;
+  int binner;
 };
 
 // Column sums out[c] (+)= sum_r g[r ldg + c] of a [rows, cols] block in one
@@ -249,6 +253,12 @@ __global__ void __launch_bounds__(256) splitk_reduce(SplitSet s0, SplitSet s1, S
   }
   const int y = (int)blockIdx.y - has_cs;
   const SplitSet &d = y == 0 ? s0 : y == 1 ? s1 : s2;
+  int64_t from = 0, to = 0;  // batch z's partials and C
+  if (gridDim.z > 1) {
+    const unsigned z = blockIdx.z, zo = z / (unsigned)d.binner, zi = z - zo * (unsigned)d.binner;
+    from = (int64_t)z * d.splits * d.n;
+    to = zo * d.bsc + zi * d.bsc2;
+  }
   typedef typename std::conditional<VEC, f4, float>::type V;
   constexpr int kW = VEC ? 4 : 1;
   constexpr int kBatch = VEC ? 4 : 8;
@@ -259,7 +269,7 @@ __global__ void __launch_bounds__(256) splitk_reduce(SplitSet s0, SplitSet s1, S
     V v[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u)
-      if (k0 + u < d.splits) v[u] = *reinterpret_cast<const V *>(d.partial + (k0 + u) * d.n + e);
+      if (k0 + u < d.splits) v[u] = *reinterpret_cast<const V *>(d.partial + from + (k0 + u) * d.n + e);
     if (d.kahan) {
 #pragma unroll
       for (int u = 0; u < kBatch; ++u)
@@ -276,7 +286,7 @@ __global__ void __launch_bounds__(256) splitk_reduce(SplitSet s0, SplitSet s1, S
     }
   }
   const int64_t p = e / d.Q, q = e - p * d.Q;
-  V *dst = reinterpret_cast<V *>(d.C + p * d.ldc + q);
+  V *dst = reinterpret_cast<V *>(d.C + to + p * d.ldc + q);
   V v = d.alpha * s;
   if (d.bias != nullptr) v = v + *reinterpret_cast<const V *>(d.bias + q);
   if (d.res != nullptr) v = v + *reinterpret_cast<const V *>(d.res + p * d.ldr + q);
@@ -381,7 +391,7 @@ __device__ __forceinline__ void bf3_tile(const Gemm &d, int tile, int batch, cha
       return FULL || (pl + 16 * i + e < d.P && ql + 16 * j < d.Q);
     };
     if (d.splits > 1) {  // plain partial product, row stride Q; splitk_reduce finishes
-      float *part = d.partial + (int64_t)split * d.P * d.Q;
+      float *part = d.partial + ((int64_t)batch * d.splits + split) * d.P * d.Q;
 #pragma unroll
       for (int i = 0; i < BI; ++i)
 #pragma unroll
@@ -477,7 +487,7 @@ bool colsum_fits(const float *g, int64_t rows, int64_t cols, int64_t ldg) {
 // reduces the set `extra` (then the launch is made even when nothing was
 // split).
 int reduce_splits(numrs_hip_ctx *ctx, const Gemm *a, const Gemm *b, const ColSum *cs = nullptr,
-                  const SplitSet *extra = nullptr) {
+                  const SplitSet *extra = nullptr, int64_t batch = 1) {
   const Gemm *g[2];
   int m = 0;
   if (a != nullptr && a->splits > 1) g[m++] = a;
@@ -489,12 +499,12 @@ int reduce_splits(numrs_hip_ctx *ctx, const Gemm *a, const Gemm *b, const ColSum
   for (int i = 0; i < m; ++i) {
     const Gemm &d = *g[i];
     set[i] = SplitSet{d.partial, d.C, d.bias, d.ldc, (int64_t)d.P * d.Q, d.Q, d.splits,
-                      d.accumulate, d.alpha, d.act, d.pre, d.res, d.ldr};
+                      d.accumulate, d.alpha, d.act, d.pre, d.res, d.ldr, 0, d.bsc, d.bsc2, d.binner};
   }
   if (extra != nullptr) set[m++] = *extra;
   for (int i = 0; i < m; ++i) {
     const SplitSet &d = set[i];
-    vec = vec && d.Q % 4 == 0 && d.ldc % 4 == 0 && numrs_hip::aligned16(d.C) &&
+    vec = vec && d.Q % 4 == 0 && d.ldc % 4 == 0 && d.bsc % 4 == 0 && d.bsc2 % 4 == 0 && numrs_hip::aligned16(d.C) &&
           numrs_hip::aligned16(d.partial) && (d.bias == nullptr || numrs_hip::aligned16(d.bias)) &&
           (d.res == nullptr || (numrs_hip::aligned16(d.res) && d.ldr % 4 == 0)) &&
           (d.pre == nullptr || numrs_hip::aligned16(d.pre));
@@ -511,7 +521,7 @@ int reduce_splits(numrs_hip_ctx *ctx, const Gemm *a, const Gemm *b, const ColSum
   }
   if (blocks > 0x7fffffff)
     return numrs_hip::fail(ctx, NUMRS_HIP_E_INVALID, "splitk_reduce: too large");
-  dim3 grid((unsigned)std::max<int64_t>(blocks, 1), (unsigned)(m + has_cs));
+  dim3 grid((unsigned)std::max<int64_t>(blocks, 1), (unsigned)(m + has_cs), (unsigned)batch);
   if (vec)
     splitk_reduce<true><<<grid, 256, 0, ctx->stream>>>(set[0], set[1], set[2], c, has_cs);
   else
@@ -875,10 +885,10 @@ int cut(int64_t k, int64_t T) {
 }
 
 // Plan for a product a, or a pair with the TN product b in the same grid,
-// over `batch` batch entries.  Batch 1: candidate tile lengths T are
+// over `batch` batch entries, all cut alike.  Candidate tile lengths T are
 // ceil(k / s) for s = 1..kMaxSplits of either product; each product is cut
 // into ceil(k / T) ranges (none empty) and the smallest estimate wins, ties
-// going to the larger tile.  Batches are not split.
+// going to the larger tile.
 Plan plan_product(numrs_hip_ctx *ctx, const Gemm &a, bool xa, bool ya, const Gemm *b,
                   int64_t batch) {
   const int64_t cus = std::max(ctx->num_cus, 1);
@@ -890,15 +900,13 @@ Plan plan_product(numrs_hip_ctx *ctx, const Gemm &a, bool xa, bool ya, const Gem
     const int64_t tb = b ? ceil_div(b->P, s.tp) * ceil_div(b->Q, s.tq) : 0;
     const int64_t kb = b ? ceil_div(b->R, kBR) : 0;
     for (int cand = 0; cand < 2 * kMaxSplits; ++cand) {
-      if (cand > 0 && batch > 1) break;
       if (cand >= kMaxSplits && !b) break;
-      const int64_t T = batch > 1 ? std::max(ka, kb)
-                                  : ceil_div(cand < kMaxSplits ? ka : kb, cand % kMaxSplits + 1);
+      const int64_t T = ceil_div(cand < kMaxSplits ? ka : kb, cand % kMaxSplits + 1);
       const int sa = cut(ka, T), sb = b ? cut(kb, T) : 1;
       const int64_t len = std::max(ceil_div(ka, sa), b ? ceil_div(kb, sb) : 0);
       double t = shape_us(s, ceil_div((ta * sa + tb * sb) * batch, cus), len);
-      if (sa > 1) t += 8.0 * sa * a.P * a.Q / kPartialBytesPerUs;
-      if (sb > 1) t += 8.0 * sb * b->P * b->Q / kPartialBytesPerUs;
+      if (sa > 1) t += 8.0 * batch * sa * a.P * a.Q / kPartialBytesPerUs;
+      if (sb > 1) t += 8.0 * batch * sb * b->P * b->Q / kPartialBytesPerUs;
       if (sa > 1 || sb > 1) t += kReduceUs;
       if (best.shape < 0 || t < best.t) best = {shape, sa, sb, t};
     }
@@ -917,16 +925,21 @@ Gemm as_shape(Gemm g, int shape) {
 }
 
 // Descriptors for a plan, with split products pointed at the context's workspace.
-// `sums`: room for the partial row sums of a split gb too (gb->sums).
-int prepare_plan(numrs_hip_ctx *ctx, const Plan &pl, Gemm &ga, Gemm *gb, bool sums = false) {
+// `sums`: room for the partial row sums of a split gb too (gb->sums).  A batch whose workspace is
+// refused (no memory, or a recording that must not grow it) runs unsplit.
+int prepare_plan(numrs_hip_ctx *ctx, const Plan &pl, int64_t batch, Gemm &ga, Gemm *gb, bool sums = false) {
   ga = as_shape(ga, pl.shape);
   if (gb != nullptr) *gb = as_shape(*gb, pl.shape);
-  const size_t na = pl.sa > 1 ? (size_t)pl.sa * ga.P * ga.Q : 0;
-  const size_t nb = gb != nullptr && pl.sb > 1 ? (size_t)pl.sb * gb->P * gb->Q : 0;
+  const size_t na = pl.sa > 1 ? (size_t)batch * pl.sa * ga.P * ga.Q : 0;
+  const size_t nb = gb != nullptr && pl.sb > 1 ? (size_t)batch * pl.sb * gb->P * gb->Q : 0;
   if (na + nb == 0) return NUMRS_HIP_OK;
   void *ws = nullptr;
   const size_t at = (na + nb + 3) & ~size_t{3}, ns = sums && nb ? (size_t)pl.sb * gb->P : 0;
-  if (int rc = numrs_hip::workspace(ctx, (at + ns) * sizeof(float), &ws)) return rc;
+  if (int rc = numrs_hip::workspace(ctx, (at + ns) * sizeof(float), &ws)) {
+    if (batch == 1) return rc;
+    (void)hipGetLastError();
+    return NUMRS_HIP_OK;
+  }
   float *base = static_cast<float *>(ws);
   if (ns) gb->sums = base + at;
   if (na) apply_splits(ga, pl.sa, base);
@@ -992,7 +1005,7 @@ int launch_one(numrs_hip_ctx *ctx, Gemm g, int64_t batch) {
   if (g.P == 0 || g.Q == 0 || batch == 0) return NUMRS_HIP_OK;
   if (tiny_fits(g, batch)) return launch_tiny(ctx, g, XRC, YRC, nullptr, batch, nullptr);
   const Plan pl = plan_product(ctx, g, XRC, YRC, nullptr, batch);
-  if (int rc = prepare_plan(ctx, pl, g, nullptr)) return rc;
+  if (int rc = prepare_plan(ctx, pl, batch, g, nullptr)) return rc;
   if (grid_tiles(g) * batch > 0x7fffffff)
     return numrs_hip::fail(ctx, NUMRS_HIP_E_INVALID, "gemm: too many tiles");
   const dim3 grid((unsigned)grid_tiles(g), (unsigned)batch);
@@ -1012,7 +1025,7 @@ int launch_one(numrs_hip_ctx *ctx, Gemm g, int64_t batch) {
     });
   }
   if (int rc = numrs_hip::check_launch(ctx, "gemm_kernel")) return rc;
-  return reduce_splits(ctx, &g, nullptr);
+  return reduce_splits(ctx, &g, nullptr, nullptr, nullptr, batch);
 }
 
 // One launch of the products ga (layout xa, ya: NT, NN or TN) and gb (TN),
@@ -1025,11 +1038,11 @@ int launch_two(numrs_hip_ctx *ctx, Gemm ga, bool xa, bool ya, Gemm gb, int64_t b
                const ColSum *sums = nullptr) {
   const Plan pl = plan_product(ctx, ga, xa, ya, &gb, batch);
   if (sums != nullptr) gb.sums = sums->out, gb.sums_acc = sums->acc;
-  if (int rc = prepare_plan(ctx, pl, ga, &gb, sums != nullptr)) return rc;
+  if (int rc = prepare_plan(ctx, pl, batch, ga, &gb, sums != nullptr)) return rc;
   SplitSet part;
   if (sums != nullptr && gb.splits > 1) {
     part = SplitSet{gb.sums, sums->out, nullptr, gb.P, gb.P, gb.P, gb.splits, sums->acc, 1.0f, 0,
-                    nullptr, nullptr, 0, 0};
+                    nullptr, nullptr, 0, 0, 0, 0, 1};
     gb.sums_acc = 0;
     extra = &part;
   }
@@ -1049,7 +1062,7 @@ int launch_two(numrs_hip_ctx *ctx, Gemm ga, bool xa, bool ya, Gemm gb, int64_t b
       gemm_pair_kernel<false, false, S><<<grid, S::NT, 0, ctx->stream>>>(ga, gb, (int)na);
   });
   if (int rc = numrs_hip::check_launch(ctx, who)) return rc;
-  return reduce_splits(ctx, &ga, &gb, cs, extra);
+  return reduce_splits(ctx, &ga, &gb, cs, extra, batch);
 }
 
 int gemm_dispatch(numrs_hip_ctx *ctx, const Gemm &g, int64_t batch, bool xrc, bool yrc) {
@@ -1284,7 +1297,7 @@ int numrs_hip::gemm_tn2_colsum(numrs_hip_ctx *ctx, const float *X, int64_t ldx, 
   // [db_rows, K] in row order, as one more set of the split reduce
   const bool by_part = db != nullptr && db_part != nullptr && db_rows >= 1 && db_rows <= (1 << 20);
   SplitSet part{db_part, db, nullptr, K, K, (int)K, (int)db_rows, acc_db, 1.0f, 0, nullptr,
-                nullptr, 0, 1};
+                nullptr, 0, 1, 0, 0, 1};
   const SplitSet *extra = by_part ? &part : nullptr;
   const bool cs_ok = db != nullptr && !by_part && colsum_fits(X, M, K, ldx);
   if (tiny_fits(ga, 1) && tiny_fits(gb, 1)) {

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from conftest import assert_contraction, rand
+from numrs_amd import Context, StepGraph
 from numrs_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
@@ -198,3 +199,78 @@ def test_left_out_terms(hip_ctx):
     got = _product(hip_ctx, np.full((M, K), x), np.full((K, N), x), 0, 0)
     ref = K * float(x) ** 2
     assert np.abs(got / ref - 1).max() < (1.01 + np.sqrt(K / 32 + 6)) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("batch,M,K,N", [(16, 256, 2048, 256), (3, 70, 5001, 333), (5, 64, 4100, 66)])
+def test_batched_splits(hip_ctx, rng, batch, M, K, N, ta, tb):
+    """Batched products of few tiles and a long reduction, cut into ranges: accumulated, at whole
+    and odd sizes, the same bits in every call."""
+    print(f"[gpu] bf3 batched splits {batch} x {M}x{K}x{N} ta={ta} tb={tb}", flush=True)
+    c = hip_ctx
+    A = rand(rng, (batch, K, M) if ta else (batch, M, K))
+    B = rand(rng, (batch, N, K) if tb else (batch, K, N))
+    C0 = rand(rng, (batch, M, N))
+    Ad, Bd = c.to_device(A), c.to_device(B)
+    got = []
+    for _ in range(2):
+        C = c.to_device(C0)
+        c.matmul_batched(Ad, Bd, C, trans_a=bool(ta), trans_b=bool(tb), accumulate=True)
+        got.append(C.numpy())
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    ref = C0 + (a.transpose(0, 2, 1) if ta else a) @ (b.transpose(0, 2, 1) if tb else b)
+    assert_contraction(got[0], ref, K, what="C")
+    assert np.array_equal(*got)
+
+
+@pytest.mark.parametrize("batch,M,K,N", [(4, 4096, 64, 64), (2, 5003, 130, 70), (3, 66, 64, 4100)])
+def test_batched_pair_splits(hip_ctx, rng, batch, M, K, N):
+    """matmul_backward over batches, one of the pair's products cut (M long: dB, N long: dA)."""
+    print(f"[gpu] bf3 batched pair splits {batch} x {M}x{K}x{N}", flush=True)
+    c = hip_ctx
+    A, B, g = rand(rng, (batch, M, K)), rand(rng, (batch, K, N)), rand(rng, (batch, M, N))
+    dA0, dB0 = rand(rng, A.shape), rand(rng, B.shape)
+    dA, dB = c.to_device(dA0), c.to_device(dB0)
+    c.matmul_backward_batched(c.to_device(g), c.to_device(A), c.to_device(B), dA, dB, accumulate=True)
+    g64 = g.astype(np.float64)
+    assert_contraction(dA.numpy(), dA0 + g64 @ B.astype(np.float64).transpose(0, 2, 1), N, what="dA")
+    assert_contraction(dB.numpy(), dB0 + A.astype(np.float64).transpose(0, 2, 1) @ g64, M, what="dB")
+
+
+@pytest.mark.parametrize("N", [24, 33])
+def test_two_level_batch_splits(hip_ctx, rng, N):
+    """Heads interleaved in B and C (two batch strides), the reduction cut; what lies between the
+    heads' outputs stays."""
+    b, H, M, K = 2, 3, 64, 3000
+    print(f"[gpu] bf3 two-level batch splits N={N}", flush=True)
+    c, lib = hip_ctx, L.load()
+    A, B = rand(rng, (b * H, K, M)), rand(rng, (b, K, H + 1, N))
+    C0 = rand(rng, (b, M, H + 1, N))
+    Ad, Bd, C = c.to_device(A), c.to_device(B), c.to_device(C0)
+    ld = (H + 1) * N
+    assert lib.numrs_hip_gemm(c.handle, Ad.ptr, M, Bd.ptr, ld, C.ptr, ld, M, K, N, 1, 0, 0.5, 0, b * H, H,
+                              H * K * M, K * M, K * ld, N, M * ld, N) == 0
+    got = C.numpy()
+    for z in range(b * H):
+        ref = 0.5 * (A[z].astype(np.float64).T @ B[z // H, :, z % H].astype(np.float64))
+        assert_contraction(got[z // H, :, z % H], ref, K, what=f"C[{z}]")
+    assert np.array_equal(got[:, :, H], C0[:, :, H])
+
+
+def test_batched_without_workspace(rng):
+    """A recording must not grow the workspace: a batch that wants one runs unsplit there."""
+    batch, M, K, N = 4, 128, 4096, 128
+    A, B = rand(rng, (batch, M, K)), rand(rng, (batch, K, N))
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    with Context(0) as c:
+        Ad, Bd, C, E = c.to_device(A), c.to_device(B), c.zeros((batch, M, N)), c.zeros((batch, M, N))
+        graph = StepGraph(c, lambda: c.matmul_batched(Ad, Bd, C))
+        try:
+            for _ in range(3):
+                C.fill(7.0)
+                graph.replay()
+                c.matmul_batched(Ad, Bd, E)  # eager: the workspace grows between the replays
+                assert_contraction(C.numpy(), ref, K, what="replayed")
+                assert_contraction(E.numpy(), ref, K, what="eager")
+        finally:
+            graph.close()
