@@ -267,13 +267,6 @@ int cross_entropy_loss_impl(numrs_hip_ctx *ctx, const float *logits, const float
                             float *seed);
 bool cross_entropy_preforms(int64_t B);
 
-// C1_z = alpha1 X1_z^T Y1_z and C2_z = alpha2 X2_z^T Y2_z (X [M,K], Y [M,N],
-// C [K,N]) for z < batch, in one launch
-// (attention's dV = P^T dO with dK = alpha dS^T Q).  Either output may be
-// null; accumulate adds into the outputs.
-int gemm_tn_pair(numrs_hip_ctx *ctx, BatchedMat X1, BatchedMat Y1, BatchedOut C1, float alpha1,
-                 BatchedMat X2, BatchedMat Y2, BatchedOut C2, float alpha2, int64_t M, int64_t K,
-                 int64_t N, int accumulate, int64_t batch, int64_t binner);
 // Two weight gradients of one left operand, C1[K,N1] = X^T Y1 and
 // C2[K,N2] = X^T Y2 (X [M,K] at row stride ldx, Y1 [M,N1], Y2 [M,N2]), in
 // one launch with a joint split plan, and the

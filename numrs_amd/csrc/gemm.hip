@@ -137,13 +137,13 @@ constexpr int kColSumClasses = 256 / kColSumLanes;  // row classes of a workgrou
 // Column groups of a [., cols] block.
 __host__ __device__ inline int64_t colsum_groups(int64_t cols) { return (cols + kColSumCols - 1) / kColSumCols; }
 
-// Threads past the first 256 of a larger workgroup only meet the barriers.
+// A workgroup of 256.
 __device__ __forceinline__ void colsum_block(const ColSum &c, int64_t blk) {
   __shared__ f4 red[256];
   const int k = threadIdx.x;
   const int j = k % kColSumLanes, rc = k / kColSumLanes;  // column chunk, row class
   const float *p = c.g + blk * kColSumCols + 4 * j;
-  const bool live = k < 256 && blk * kColSumCols + 4 * j < c.cols;
+  const bool live = blk * kColSumCols + 4 * j < c.cols;
   f4 s = {0.0f, 0.0f, 0.0f, 0.0f};
   for (int64_t r0 = rc; live && r0 < c.rows; r0 += kColSumClasses * 16) {
     f4 v[16];
@@ -155,7 +155,7 @@ __device__ __forceinline__ void colsum_block(const ColSum &c, int64_t blk) {
 #pragma unroll
     for (int u = 0; u < 16; ++u) s += v[u];
   }
-  if (k < 256) red[k] = s;  // k = kColSumLanes * class + chunk
+  red[k] = s;  // k = kColSumLanes * class + chunk
   __syncthreads();
   // 64 partials: chunk t % lanes, classes 4 (t / lanes) .. + 3, added in order
   f4 t = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -186,55 +186,21 @@ __device__ __forceinline__ int64_t colsum_group(int b, int n, int64_t m) {
   return idx < (m >> 3) ? (b & 7) * (m >> 3) + idx : -1;
 }
 
-// Adds the splits' values v[0..n) to the running sum s in split order, plain
-// or compensated (kahan): the operations of splitk_reduce's loop, for the
-// reductions made inside a product's launch (tiny_tile).
-template <class V, int N>
-__device__ __forceinline__ void add_splits(int kahan, V &s, V &comp, const V (&v)[N], int n) {
-  if (kahan) {
-#pragma unroll
-    for (int u = 0; u < N; ++u)
-      if (u < n) {
-        const V y = v[u] - comp;
-        const V t = s + y;
-        comp = (t - s) - y;
-        s = t;
-      }
-  } else {
-#pragma unroll
-    for (int u = 0; u < N; ++u)
-      if (u < n) s += v[u];
-  }
-}
-
-// The end of a split reduction at C[p, q..]: alpha, bias, residual,
-// accumulate, activation (pre-activation stored first) -- splitk_reduce's
-// epilogue, operation for operation.  Takes the set's fields one by one (a
-// reference to a kernel argument, once inlined, had fields copied to private
-// memory).  splitk_reduce keeps its own copy of this arithmetic: with these
-// helpers inlined its set selection was promoted to LDS.
-template <class V>
-__device__ __forceinline__ void finish_split(float *C, int64_t ldc, const float *bias,
-                                             const float *res, int64_t ldr, int acc, float alpha,
-                                             int act, float *pre, int64_t p, int64_t q, V s) {
-  V *dst = reinterpret_cast<V *>(C + p * ldc + q);
-  V v = alpha * s;
-  if (bias != nullptr) v = v + *reinterpret_cast<const V *>(bias + q);
-  if (res != nullptr) v = v + *reinterpret_cast<const V *>(res + p * ldr + q);
-  v = acc ? *dst + v : v;
-  if (act) {
-    if (pre != nullptr) *reinterpret_cast<V *>(pre + p * ldc + q) = v;
-    if constexpr (std::is_same<V, f4>::value) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = act_value(act, v[e]);
-    } else {
-      v = act_value(act, v);
-    }
+// The end of a split reduction at C[p, q] made inside a product's launch (tiny_tile): alpha, bias,
+// residual, accumulate, activation (pre-activation stored first), as splitk_reduce's epilogue,
+// operation for operation.
+__device__ __forceinline__ void finish_split(float *C, const Gemm &d, int64_t p, int64_t q, float s) {
+  float *dst = C + p * d.ldc + q;
+  float v = d.alpha * s;
+  if (d.bias != nullptr) v = v + d.bias[q];
+  if (d.res != nullptr) v = v + d.res[p * d.ldr + q];
+  v = d.accumulate ? *dst + v : v;
+  if (d.act) {
+    if (d.pre != nullptr) d.pre[p * d.ldc + q] = v;
+    v = act_value(d.act, v);
   }
   *dst = v;
 }
-#define NRS_FINISH_SPLIT(d, p, q, s) \
-  finish_split((d).C, (d).ldc, (d).bias, (d).res, (d).ldr, (d).acc, (d).alpha, (d).act, (d).pre, p, q, s)
 
 // Splits are added in order s = 0, 1, ... (deterministic); the loads of a
 // batch of splits are issued before its ordered adds.  With column sums
@@ -454,7 +420,7 @@ __global__ void __launch_bounds__(S::NT, kWavesPerSimd<S>) gemm_kernel(Gemm d) {
 // Two products in one grid: logical tiles [0, tiles_a) belong to `a`, the
 // rest to `b`, which is TN.  matmul_backward: dA = dC B^T (NT) with dB =
 // A^T dC; the Linear backward: dx = g W (NN) with dW = g^T x; two weight
-// gradients, or attention's dV = P^T dO with dK = alpha dS^T Q (TN).
+// gradients (TN).
 template <bool XA, bool YA, class S, bool SUMS = false>
 __global__ void __launch_bounds__(S::NT, kWavesPerSimd<S>) gemm_pair_kernel(Gemm a, Gemm b,
                                                                             int tiles_a) {
@@ -476,7 +442,7 @@ void apply_splits(Gemm &g, int splits, float *partial) {
 
 // Whether the column sums of g [rows, cols] (row stride ldg) can ride in the
 // split-reduce launch: float4 column groups and at most 8192 rows (a
-// workgroup walks every row of its 16 columns).
+// workgroup walks every row of its eight columns).
 bool colsum_fits(const float *g, int64_t rows, int64_t cols, int64_t ldg) {
   return cols % 4 == 0 && ldg % 4 == 0 && numrs_hip::aligned16(g) && rows <= 8192 &&
          cols / kColSumCols <= 0x7ffffff0;
@@ -556,7 +522,7 @@ constexpr int kTinyMaxR = 4096;  // at most four load batches per wave
 // FUSE (batch 1, d.arrive set for a split product): a split stores its
 // partial at device scope and arrives at its output block's counter; the
 // last of the block's splits adds the block's partials in split order with
-// splitk_reduce's arithmetic (add_splits, finish_split) and sets the counter
+// splitk_reduce's arithmetic (finish_split) and sets the counter
 // back to zero -- no reduce launch, and no workgroup waits for another.
 template <bool XRC, bool YRC, int U, bool FUSE = false>
 __device__ __forceinline__ void tiny_tile(const Gemm &d, int tile, int batch) {
@@ -661,16 +627,17 @@ __device__ __forceinline__ void tiny_tile(const Gemm &d, int tile, int batch) {
         if (pp < d.P && qq < d.Q) {
           const int64_t n = (int64_t)d.P * d.Q, e = (int64_t)pp * d.Q + qq;
           const __amdgpu_buffer_rsrc_t rs = numrs_hip::dev_rsrc(d.partial, (int64_t)d.splits * n * 4);
-          float sum = 0.0f, comp = 0.0f;
+          float sum = 0.0f;
           for (int k0 = 0; k0 < d.splits; k0 += 8) {
             float v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u)
               if (k0 + u < d.splits) v[u] = numrs_hip::ld_dev1(rs, (int)(4 * ((k0 + u) * n + e)));
-            add_splits(0, sum, comp, v, d.splits - k0);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+              if (k0 + u < d.splits) sum += v[u];
           }
-          finish_split(C, d.ldc, d.bias, d.res, d.ldr, d.accumulate, d.alpha, d.act, d.pre,
-                       (int64_t)pp, (int64_t)qq, sum);
+          finish_split(C, d, pp, qq, sum);
         }
       }
     }
@@ -1239,45 +1206,6 @@ int numrs_hip::gemm_nn_tn_pair(numrs_hip_ctx *ctx, BatchedMat X, BatchedMat Y1, 
   return launch_two(ctx, ga, true, false, gb, batch, nullptr, nullptr, who);
 }
 
-int numrs_hip::gemm_tn_pair(numrs_hip_ctx *ctx, BatchedMat X1, BatchedMat Y1, BatchedOut C1,
-                            float alpha1, BatchedMat X2, BatchedMat Y2, BatchedOut C2,
-                            float alpha2, int64_t M, int64_t K, int64_t N, int accumulate,
-                            int64_t batch, int64_t binner) {
-  const char *who = "gemm_tn_pair";
-  if (int rc = check_dims(ctx, who, batch, M, K, N)) return rc;
-  if (binner < 1 || binner > std::max<int64_t>(batch, 1))
-    return numrs_hip::fail(ctx, NUMRS_HIP_E_INVALID, "%s: batch_inner %lld", who, (long long)binner);
-  if (batch == 0 || N == 0 || K == 0 || (C1.p == nullptr && C2.p == nullptr)) return NUMRS_HIP_OK;
-  if ((C1.p && (X1.p == nullptr || Y1.p == nullptr)) || (C2.p && (X2.p == nullptr || Y2.p == nullptr)))
-    return numrs_hip::fail(ctx, NUMRS_HIP_E_INVALID, "%s: null input", who);
-  // C[K,N] = alpha X^T Y with X [M,K], Y [M,N]: P=K, Q=N, R=M, both operands
-  // output-contiguous.
-  auto tn = [&](BatchedMat X, BatchedMat Y, BatchedOut C, float alpha) {
-    Gemm g = make(X.p, Y.p, C.p, X.ld, Y.ld, C.ld, X.so, Y.so, C.so, K, N, M, accumulate);
-    g.bsx2 = X.si, g.bsy2 = Y.si, g.bsc2 = C.si;
-    g.binner = (int)binner;
-    g.alpha = alpha;
-    return g;
-  };
-  if (M == 0) {  // an empty reduction leaves zeros (or the accumulated values)
-    for (int64_t z = 0; z < batch && !accumulate; ++z) {
-      const int64_t zo = z / binner, zi = z - zo * binner;
-      for (const BatchedOut *C : {&C1, &C2})
-        if (C->p)
-          for (int64_t r = 0; r < K; ++r)
-            if (int rc = numrs_hip_fill(ctx, C->p + zo * C->so + zi * C->si + r * C->ld, N, 0.0f))
-              return rc;
-    }
-    return NUMRS_HIP_OK;
-  }
-  const Gemm ga = C1.p ? tn(X1, Y1, C1, alpha1) : Gemm{}, gb = C2.p ? tn(X2, Y2, C2, alpha2) : Gemm{};
-  if (C1.p == nullptr) return gemm_dispatch(ctx, gb, batch, false, false);
-  if (C2.p == nullptr) return gemm_dispatch(ctx, ga, batch, false, false);
-  if (batch > 1 && tiny_fits(ga, batch) && tiny_fits(gb, batch))
-    return launch_tiny(ctx, ga, false, false, &gb, batch, nullptr);
-  return launch_two(ctx, ga, false, false, gb, batch, nullptr, nullptr, who);
-}
-
 int numrs_hip::gemm_tn2_colsum(numrs_hip_ctx *ctx, const float *X, int64_t ldx, int64_t M,
                                int64_t K, const float *Y1, int64_t ldy1, int64_t N1, float *C1,
                                int acc1, const float *Y2, int64_t ldy2, int64_t N2, float *C2,
@@ -1289,7 +1217,7 @@ int numrs_hip::gemm_tn2_colsum(numrs_hip_ctx *ctx, const float *X, int64_t ldx, 
       M <= 0 || K <= 0 || N1 <= 0 || N2 <= 0)
     return numrs_hip::fail(ctx, NUMRS_HIP_E_INVALID, "%s: null or empty operand", who);
   // C[K,N] = X^T Y with X [M,K], Y [M,N]: P=K, Q=N, R=M (both operands
-  // output-contiguous), as gemm_tn_pair.
+  // output-contiguous).
   Gemm ga = make(X, Y1, C1, ldx, ldy1, N1, 0, 0, 0, K, N1, M, acc1);
   Gemm gb = make(X, Y2, C2, ldx, ldy2, N2, 0, 0, 0, K, N2, M, acc2);
   ColSum cs{X, db, M, K, ldx, acc_db, nullptr};
@@ -1358,8 +1286,8 @@ int numrs_hip_linear_backward(numrs_hip_ctx *ctx, const float *g, const float *x
       if (int rc = numrs_hip_fill(ctx, dW, out * in, 0.0f)) return rc;
   } else {
     // db = column sums of g (CORRECT mode), formed by the pair's own launch
-    // (tiny products) or by the launch that reduces its splits, rather than
-    // by two launches of their own
+    // (launch_pair: tiny products' own workgroups, or the dW product's tiles)
+    // or, without dx or dW, by a launch of their own
     ColSum cs{g, db, T, out, out, acc_db};
     const bool want_db = db != nullptr && mode == NUMRS_HIP_UNBROADCAST_CORRECT;
     bool db_done = false;
