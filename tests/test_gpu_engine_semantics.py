@@ -159,9 +159,9 @@ def test_layernorm_with_gamma_as_beta():
 @pytest.mark.parametrize("S", [128, 256])
 @pytest.mark.parametrize("mode", ["dq", "dk", "dv", "self"])
 def test_attention_single_head(S, mode):
-    """B = H = 1, dh = 64: dQ = dS K and dK = dS^T Q are single 128 x 64 or
-    256 x 64 products with an S-long reduction, which split it (the split
-    partials must not overwrite dS)."""
+    """B = H = 1, dh = 64 and one or two of the three gradients: dQ = dS K and dK =
+    dS^T Q as single products with an S-long reduction, cut in two at S = 256
+    (the partials must not overwrite dS)."""
     print(f"[gpu] attention single head S={S} mode={mode}", flush=True)
     D = 64
     rng = np.random.default_rng(29 + S)

@@ -1,18 +1,17 @@
-"""Split-K partials added inside the products' own launch (the default,
-numrs_hip_set_split_reduction FUSED, for the 128 x 64 streamed tiles and the
-16 x 16 tiny blocks) against one more launch after them (SEPARATE): the same
-bits, for the Linear backward pairs of the C4 block, for matmul_backward
-shapes whose weight-side product splits, for C1's first layer, and for the
-C5 forecaster's paired LSTM weight gradients.  (Products
-on the 256 x 128 tiles keep the separate launch in both modes.)  The fused
-form's arrival counters are reset by the launches themselves, so
-back-to-back calls and replays of a recorded graph must each be whole."""
+"""Split-K partials of small products (at most 2^24 multiply-adds, 16 x 16 blocks) added
+inside their own launch (the default, numrs_hip_set_split_reduction FUSED) against one more
+launch after them (SEPARATE): the same bits, for Linear and matmul gradient pairs with
+either or both products cut, the first layer of a batch-64 MLP and the head of the LSTM
+forecaster.  The arrival counters are reset by the launches themselves, so back-to-back
+calls and replays of a recorded graph must each be whole.  Larger products take the separate
+launch in both modes: there both modes are compared with float64 as well."""
 import numpy as np
 import pytest
 
 import numrs_amd as nr
 from numrs_amd import StepGraph, Tensor, nn
 from numrs_amd import _lib as L
+from conftest import assert_contraction
 from oracle import lstm_oracle as LO
 
 pytestmark = pytest.mark.gpu
@@ -30,13 +29,31 @@ def _linear_bwd(c, gd, xd, Wd, outs, T, fin, fout, acc):
     assert rc == 0
 
 
-# The C4 block's four Linear shapes (all split their weight gradient; the
-# packed q/k/v projection splits dx too), a small-tile product and a shape
-# whose bias columns end on a partial column group.
-@pytest.mark.parametrize("T,fin,fout", [(4096, 2048, 512), (4096, 512, 2048), (4096, 512, 512),
-                                        (4096, 512, 1536), (2048, 256, 256), (8192, 64, 100)])
+def _tiny_splits(blocks, R, cus=256):
+    """Ranges of a small product's reduction: enough for a workgroup to a CU, of at least four
+    32-wide tiles each."""
+    tiles = -(-R // 32)
+    n = min(-(-cus // blocks), tiles // 4, 32)
+    return -(-tiles // -(-tiles // n)) if n > 1 else 1
+
+
+def _blocks(P, Q):
+    return -(-P // 16) * -(-Q // 16)
+
+
+# Small pairs, (ranges of dx, of dW): (1, 2), (1, 4), (1, 5), (5, 1), (2, 2), and ragged (1, 5),
+# (3, 3).  Large ones: the C4 block's four Linear shapes (all split their weight gradient; the
+# packed q/k/v projection splits dx too), and two on 64 x 64 tiles.
+TINY = [(300, 64, 64), (1000, 16, 16), (900, 16, 33), (16, 16, 700), (300, 16, 300), (901, 5, 17), (397, 9, 389)]
+
+
+@pytest.mark.parametrize("T,fin,fout", TINY + [(4096, 2048, 512), (4096, 512, 2048), (4096, 512, 512),
+                                               (4096, 512, 1536), (2048, 256, 256), (8192, 64, 100)])
 def test_linear_backward_fused_equals_separate(hip_ctx, rng, T, fin, fout):
     print(f"[gpu] fused split reduction: linear backward T={T} in={fin} out={fout}", flush=True)
+    if T * fin * fout <= 1 << 24:  # the shape does what it is here for
+        blocks = _blocks(T, fin) + _blocks(fout, fin)
+        assert max(_tiny_splits(blocks, fout), _tiny_splits(blocks, T)) > 1
     c = hip_ctx
     x = rng.standard_normal((T, fin), dtype=np.float32)
     W = rng.standard_normal((fout, fin), dtype=np.float32)
@@ -58,13 +75,19 @@ def test_linear_backward_fused_equals_separate(hip_ctx, rng, T, fin, fout):
                 got[mode] = vals
             for a, b, name in zip(got["separate"], got["fused"], ("dx", "dW", "db")):
                 assert np.array_equal(a, b), f"{name} acc={acc}"
+            g64, base = g.astype(np.float64), [a * p for a, p in zip(acc, prev)]
+            dx, dW, db = got["fused"]
+            assert_contraction(dx, base[0] + g64 @ W.astype(np.float64), fout, what=f"dx {acc}")
+            assert_contraction(dW, base[1] + g64.T @ x.astype(np.float64), T, what=f"dW {acc}")
+            assert_contraction(db, base[2] + g64.sum(0), T, what=f"db {acc}")
     finally:
         c.set_split_reduction("fused")
 
 
-# matmul_backward shapes whose dB = A^T dC runs over a long reduction (M):
-# the planner cuts it into split-K ranges beside the unsplit dA tiles.
-@pytest.mark.parametrize("M,K,N", [(8192, 512, 512), (16384, 256, 512), (4096, 1024, 256)])
+# matmul_backward pairs: small ones with dB = A^T dC cut over M, dA over N, or both; large ones
+# with dB cut beside the unsplit dA tiles.
+@pytest.mark.parametrize("M,K,N", [(1000, 16, 16), (16, 16, 1000), (300, 16, 300), (397, 9, 389),
+                                   (8192, 512, 512), (16384, 256, 512), (4096, 1024, 256)])
 def test_matmul_backward_fused_equals_separate(hip_ctx, rng, M, K, N):
     print(f"[gpu] fused split reduction: matmul_backward {M}x{K}x{N}", flush=True)
     c = hip_ctx
@@ -72,12 +95,18 @@ def test_matmul_backward_fused_equals_separate(hip_ctx, rng, M, K, N):
     B = c.to_device(rng.standard_normal((K, N), dtype=np.float32))
     dC = c.to_device(rng.standard_normal((M, N), dtype=np.float32))
     got = {}
+    if M * K * N <= 1 << 24:
+        blocks = _blocks(M, K) + _blocks(K, N)
+        assert max(_tiny_splits(blocks, N), _tiny_splits(blocks, M)) > 1
     try:
-        for mode in ("separate", "fused"):
+        for mode in ("separate", "fused", "fused"):  # fused twice: counters back at zero
             c.set_split_reduction(mode)
             dA, dB = c.empty((M, K)), c.empty((K, N))
             c.matmul_backward(dC, A, B, dA, dB)
-            got[mode] = (dA.numpy(), dB.numpy())
+            vals = (dA.numpy(), dB.numpy())
+            for a, b, name in zip(got.get(mode, vals), vals, ("dA", "dB")):
+                assert np.array_equal(a, b), f"second fused call {name}"
+            got[mode] = vals
     finally:
         c.set_split_reduction("fused")
     assert np.array_equal(got["separate"][0], got["fused"][0]), "dA"
@@ -126,8 +155,8 @@ def test_tiny_split_fused_equals_separate(hip_ctx, rng, what):
 
 def test_lstm_forecaster_fused_equals_separate(hip_ctx, monkeypatch):
     """C5 end to end: the head Linear's split product (tiny blocks) reduces
-    in its own launch; the layers' paired weight gradients (a 128 x 64 grid
-    that leaves slots free) keep the separate reduce in both modes."""
+    in its own launch; the layers' paired weight gradients take the separate
+    reduce in both modes."""
     print("[gpu] fused split reduction: C5 forecaster", flush=True)
     nr.set_default_context(hip_ctx)
     monkeypatch.setattr(nn.LSTMForecaster, "fuse_stack", True)
@@ -154,14 +183,13 @@ def test_lstm_forecaster_fused_equals_separate(hip_ctx, monkeypatch):
         assert np.array_equal(v, fus[name]), name
 
 
-def test_fused_linear_backward_graph_replays(hip_ctx, rng):
-    """A fused Linear backward (C4's 512 -> 512 layer, small tiles, dW split)
-    recorded into a graph: each replay, with new g uploaded and eager fused
-    calls of the same shape in between, equals an eager call on the same
-    inputs."""
-    print("[gpu] fused split reduction: graph replays", flush=True)
+@pytest.mark.parametrize("T,fin,fout", [(1000, 16, 16), (16, 16, 700), (397, 9, 389), (4096, 512, 512)])
+def test_fused_linear_backward_graph_replays(hip_ctx, rng, T, fin, fout):
+    """A Linear backward with split products (small: dW, dx, both; and a large pair)
+    recorded into a graph: each replay, with new g uploaded and eager calls of the
+    same shape in between, equals an eager call on the same inputs."""
+    print(f"[gpu] fused split reduction: graph replays T={T} in={fin} out={fout}", flush=True)
     c = hip_ctx
-    T, fin, fout = 4096, 512, 512
     x = c.to_device(rng.standard_normal((T, fin), dtype=np.float32))
     W = c.to_device(rng.standard_normal((fout, fin), dtype=np.float32))
     g = c.to_device(rng.standard_normal((T, fout), dtype=np.float32))

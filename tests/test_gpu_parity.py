@@ -151,15 +151,13 @@ def test_matmul_backward_baseline_sizes(hip_ctx, rng, M, K, N):
     assert_bits(dB2.numpy(), gb * 2, "dB linearity")
 
 
-# Streamed large-tile path (256 x 128 workgroup tiles, DMA ring): taken for
-# aligned products with at least one such tile per CU.  Batches of 256 x 128
-# products reach the 256-tile threshold at small sizes; reductions of 1..7
-# and 32 tiles cover every prologue/tail case of the three-stage ring.
+# Batched products on 256 x 128 tiles, one per CU: reductions of 1..7 and 32
+# tiles of 32 steps, every case of the product loop's prologue and tail.
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192, 224, 1024])
 def test_matmul_streamed_batched(hip_ctx, rng, ta, tb, K):
     batch, M, N = 128, 256, 256
-    say(f"streamed matmul batch={batch} M={M} K={K} N={N} ta={ta} tb={tb}")
+    say(f"batched matmul batch={batch} M={M} K={K} N={N} ta={ta} tb={tb}")
     A = rand(rng, (batch, K, M) if ta else (batch, M, K))
     B = rand(rng, (batch, N, K) if tb else (batch, K, N))
     C0 = rand(rng, (batch, M, N))
@@ -170,17 +168,17 @@ def test_matmul_streamed_batched(hip_ctx, rng, ta, tb, K):
     a64 = A.astype(np.float64).transpose(0, 2, 1) if ta else A.astype(np.float64)
     b64 = B.astype(np.float64).transpose(0, 2, 1) if tb else B.astype(np.float64)
     ref = C0.astype(np.float64) + a64 @ b64
-    assert_contraction(C.numpy(), ref, K, what="streamed C += A B")
+    assert_contraction(C.numpy(), ref, K, what="batched C += A B")
 
 
 # Batched products with [256, 64] outputs per batch (attention's per-head
-# shape at C4): the planner takes the 64 x 64 mini tile, three workgroups per
-# CU; reductions of 1, 3 and 8 tiles cover the ring's prologue cases.
+# shape at C4): 128 x 64 tiles, one per CU, over reductions of 1, 3 and 8 tiles
+# of 32 steps; the gradient pair on 256 x 128 or 128 x 64 tiles.
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("K", [32, 96, 256])
 def test_matmul_streamed_batched_mini(hip_ctx, rng, ta, tb, K):
     batch, M, N = 128, 256, 64
-    say(f"streamed mini matmul batch={batch} M={M} K={K} N={N} ta={ta} tb={tb}")
+    say(f"batched narrow matmul batch={batch} M={M} K={K} N={N} ta={ta} tb={tb}")
     A = rand(rng, (batch, K, M) if ta else (batch, M, K))
     B = rand(rng, (batch, N, K) if tb else (batch, K, N))
     C0 = rand(rng, (batch, M, N))
@@ -191,7 +189,7 @@ def test_matmul_streamed_batched_mini(hip_ctx, rng, ta, tb, K):
     a64 = A.astype(np.float64).transpose(0, 2, 1) if ta else A.astype(np.float64)
     b64 = B.astype(np.float64).transpose(0, 2, 1) if tb else B.astype(np.float64)
     ref = C0.astype(np.float64) + a64 @ b64
-    assert_contraction(C.numpy(), ref, K, what="mini C += A B")
+    assert_contraction(C.numpy(), ref, K, what="narrow C += A B")
     # the matmul_backward pair at the same per-batch shape (dA NT + dB TN)
     dC = rand(rng, (batch, M, N))
     A2, B2 = rand(rng, (batch, M, K)), rand(rng, (batch, K, N))
@@ -204,10 +202,10 @@ def test_matmul_streamed_batched_mini(hip_ctx, rng, ta, tb, K):
 
 @pytest.mark.parametrize("acc", [False, True])
 def test_matmul_backward_streamed(hip_ctx, rng, acc):
-    """matmul_backward through the streamed pair kernel (dA NT + dB TN tiles
-    in one grid) at a batched shape whose tile count reaches the threshold."""
+    """matmul_backward as one pair launch (dA NT + dB TN tiles in one grid)
+    over a batch, dB's reduction over M cut into ranges."""
     batch, M, K, N = 4, 2048, 1024, 256
-    say(f"streamed matmul_backward batch={batch} M={M} K={K} N={N} acc={acc}")
+    say(f"batched matmul_backward batch={batch} M={M} K={K} N={N} acc={acc}")
     A, B, dC = rand(rng, (batch, M, K)), rand(rng, (batch, K, N)), rand(rng, (batch, M, N))
     ga0 = rand(rng, (batch, M, K)) if acc else np.zeros((batch, M, K), np.float32)
     gb0 = rand(rng, (batch, K, N)) if acc else np.zeros((batch, K, N), np.float32)
@@ -235,8 +233,7 @@ def test_matmul_forward(hip_ctx, rng, ta, tb, M, K, N):
     assert_contraction(C.numpy(), ref, K)
 
 
-# (32, 256, 128, 256): 256 tiles of 128 x 64 over the batch -- the batched
-# small-tile streamed pair.
+# (32, 256, 128, 256): 512 tiles of 128 x 64 over the batch, two per CU.
 @pytest.mark.parametrize("bt,M,K,N", [(6, 40, 64, 72), (32, 256, 128, 256)])
 def test_matmul_backward_batched(hip_ctx, rng, bt, M, K, N):
     say(f"matmul_backward_batched bt={bt} M={M} K={K} N={N}")
@@ -867,12 +864,11 @@ def test_matmul_forward_split_k_long_reduction(hip_ctx, rng):
 
 
 # (4096, 512, 2048), (4096, 2048, 512), (4096, 512, 512) and (4096, 512, 1536)
-# (the packed q/k/v projection) are the C4 block's Linear shapes: the streamed
-# 256 x 128 path with split-K ranges planned per product (dx and dW in one
-# grid, each reduced in split order).  The bias gradient (CORRECT mode) is
-# formed by the split-reduce launch for float4 columns and up to 8192 rows:
-# (8192, 64, 100) ends on a partial 16-column group; (9000, 32, 64) and
-# (130, 96, 18) take the two-pass column reduce.
+# (the packed q/k/v projection) are the C4 block's Linear shapes: 128 x 128 and
+# 256 x 128 tiles with split-K ranges planned per product (dx and dW in one
+# grid, each reduced in split order), (8192, 64, 100) and (9000, 32, 64) 64 x 64
+# tiles.  The bias gradient (CORRECT mode) comes from the dW product's tiles, or
+# from the tiny kernel's own workgroups ((64, ...), (130, 96, 18), (33, 17, 5)).
 @pytest.mark.parametrize("T,fin,fout", [(64, 784, 128), (64, 128, 10), (4096, 512, 2048),
                                         (4096, 2048, 512), (4096, 512, 512), (4096, 512, 1536),
                                         (8192, 64, 100), (9000, 32, 64), (130, 96, 18),
@@ -980,10 +976,10 @@ def test_linear_relu_forward_backward(hip_ctx, rng, T, fin, fout):
 
 
 # y = res + (x W^T + b) with the residual in the epilogue of each GEMM path:
-# tiny (64, 784, 128) and (130, 96, 18), streamed (4096, 512, 512), streamed
-# with split-K (4096, 2048, 512: the epilogue runs in the split reduction),
-# the wide 128 x 192 tile (4096, 512, 1536), the 128 x 128 path (1000, 300,
-# 136).  Bit for bit the Linear forward followed by an add; also with res
+# tiny (64, 784, 128; split: the epilogue runs in its last split) and (130, 96,
+# 18), 128 x 64 tiles (4096, 512, 512), 256 x 128 (4096, 512, 1536), split 128 x
+# 128 (4096, 2048, 512) and 64 x 64 (1000, 300, 136), whose epilogue runs in the
+# split reduction.  Bit for bit the Linear forward followed by an add; also with res
 # aliasing y.
 @pytest.mark.parametrize("T,fin,fout", [(64, 784, 128), (130, 96, 18), (4096, 512, 512),
                                         (4096, 2048, 512), (4096, 512, 1536), (1000, 300, 136)])
@@ -1008,10 +1004,9 @@ def test_linear_residual_forward(hip_ctx, rng, T, fin, fout):
 
 
 # Linear followed by GELU as one op, the pre-activation stored by the
-# epilogue: tiny (64, 784, 128) and (33, 17, 5), streamed (4096, 512, 2048:
-# the C4 FFN's first projection), streamed with split-K (4096, 2048, 512),
-# the wide 128 x 192 tile (4096, 512, 1536), the 128 x 128 path (1000, 300,
-# 136).  Bit for bit the two-op composition.
+# epilogue: tiny (64, 784, 128; split) and (33, 17, 5), 256 x 128 tiles (4096,
+# 512, 2048: the C4 FFN's first projection) and (4096, 512, 1536), split 128 x 128
+# (4096, 2048, 512) and 64 x 64 (1000, 300, 136).  Bit for bit the two-op composition.
 @pytest.mark.parametrize("T,fin,fout", [(64, 784, 128), (33, 17, 5), (4096, 512, 2048),
                                         (4096, 2048, 512), (4096, 512, 1536), (1000, 300, 136)])
 def test_linear_gelu_forward_backward(hip_ctx, rng, T, fin, fout):

@@ -23,11 +23,11 @@ def _mha_ref(q, k, v, B, S, H):
     return P, Q, K, V
 
 
-# (16, 256, 8, 512) is the C4 shape: 128 heads, enough 128 x 64 tiles for the
-# batched streamed products (dQ and dK as one pair launch).  Head size 64 with
-# S a multiple of 128 (up to 512) takes the fused row-block kernels (Q K^T +
-# softmax, dO V^T + softmax backward); S = 128, 384, 512 cover their other
-# column-block counts.
+# (16, 256, 8, 512) is the C4 shape, on eight row groups of 16 a workgroup, (3, 256, 8,
+# 512) on four.  The others are below the kernels' 32 workgroups: their forwards take
+# the kernel (heads up to 64, S <= 128 or whole blocks of 128 up to 512) but for (1, 7, 1,
+# 5), whose head size is no multiple of 8; their backwards, here without the forward's
+# output, the GEMMs.
 @pytest.mark.parametrize("B,S,H,D", [(2, 40, 4, 64), (1, 7, 1, 5), (3, 256, 8, 512),
                                      (16, 256, 8, 512), (2, 128, 2, 128), (1, 384, 1, 64),
                                      (1, 512, 2, 128)])
@@ -59,8 +59,8 @@ def test_attention_forward_backward(hip_ctx, B, S, H, D):
 @pytest.mark.parametrize("acc", [0, 1])
 def test_attention_strided_packed_qkv(hip_ctx, B, S, H, D, acc):
     """q, k, v (and dq, dk, dv) as the column blocks of one packed [B*S, 3D]
-    buffer (row stride 3D): the fused row-block path (dh = 64, S % 128 == 0)
-    and the GEMM fallback, written and accumulated."""
+    buffer (row stride 3D): the attention kernels, and the GEMMs in the smaller
+    shapes' backward, written and accumulated."""
     from numrs_amd import _lib as L
     print(f"[gpu] attention strided B={B} S={S} H={H} D={D} acc={acc}", flush=True)
     rng = np.random.default_rng(3 * B + S)
@@ -96,10 +96,10 @@ def test_attention_strided_packed_qkv(hip_ctx, B, S, H, D, acc):
 @pytest.mark.parametrize("acc", [0, 1])
 def test_attention_backward_with_output(hip_ctx, B, S, H, D, acc):
     """numrs_hip_attention_backward_out_strided on the packed [B*S, 3D] layout:
-    given the forward's output, dh = 64 with S = 256 (two row blocks per head)
-    or S = 128 (one) runs the query-row and key-row kernels when nothing
-    accumulates; S = 384, S = 40 and acc = 1 take the row-block or GEMM path.
-    Each grad against float64, and a second call returns the same bits."""
+    given the forward's output, the query-row and key-row kernels (16 x 8 heads),
+    both in one launch (fewer workgroups: 3 x 8 heads, S = 128 and 40) or the GEMMs
+    (one head of S = 384).  Each grad against float64, and a second call returns
+    the same bits."""
     from numrs_amd import _lib as L
     print(f"[gpu] attention backward with output B={B} S={S} H={H} D={D} acc={acc}",
           flush=True)
