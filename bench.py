@@ -1536,6 +1536,8 @@ def main() -> int:
                    "M": M, "K": K, "N": N, "flops_per_step": head["flops"],
                    "operand_sets": head["sets"], "sample_ok": head["sample_ok"],
                    "device": arch, "cus": n_cus},
+        # peak and frac are the metric's, of the fp32 MFMA roofline; the kernel's own ceiling
+        # is frac_of_bf16_mfma_over_six
         "roofline": {"bound": "mfma", "kernel": HEAD_KERNEL,
                      "achieved": round(achieved_tf, 3), "peak": PEAK_FP32_MFMA_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved_tf / PEAK_FP32_MFMA_TFLOPS, 4),

@@ -2,9 +2,8 @@
 //
 // An fp32 value is the sum of three bf16 values (Henry, Tang and Heinecke, "Leveraging the
 // bfloat16 artificial intelligence datatype for higher-precision computations", ARITH 2019),
-// x = h + m + l with h = bf16(x),
-// m = bf16(x - h), l = x - h - m (round to nearest even; both differences are exact, and
-// what is left after two roundings fits bf16's 8 bits).  Operands are split times 2^16, and
+// x = h + m + l with h = bf16(x), m = bf16(x - h), l = x - h - m (round to nearest even; both
+// differences are exact, and what is left after two roundings fits bf16's 8 bits).  Operands are split times 2^16, and
 // the sums multiplied by 2^-32: every fp32 value, the subnormal ones too, is then a multiple
 // of bf16's smallest subnormal, 2^-133, and the split exact (conversion and MFMA keep bf16
 // subnormals: measured).  A product is
@@ -16,11 +15,13 @@
 // 1.5e-7, where v_mfma_f32_32x32x2f32 with totals every 96 steps has 1.9 | 1.9 | 2.0e-7.
 //
 // What bounds it: gfx950's bf16 MFMA rate is 2.5 PFLOP/s against 157 TFLOP/s for fp32
-// MFMAs, so six of them take 0.38 of the time at nominal rates.  On N(0, 1) data the card
-// lowers its clock under them (about 2.0 GHz; the same launches on zeros run 1.36 times as
-// fast), and [4096, 2048] x [2048, 4096] runs at 176-184 TFLOP/s of fp32 work = 1.1 PFLOP/s
-// of bf16 (hipBLASLt's plain bf16 product of that size: 1.14; the fp32 MFMA kernel that
-// this replaced: 142 TFLOP/s).
+// MFMAs, so six of them take 0.38 of the time at nominal rates.  The matrix units are busy
+// for half of the 256 x 128 tile's cycles: a SIMD's two waves also issue 2.7 other VALU
+// instructions for each MFMA (the splits, the sums of 32 steps), which takes two thirds of
+// the MFMAs' time and is covered by them in part only.  On N(0, 1) data the clock is 2.1 GHz;
+// on zeros, at 2.4, the same launches run 1.09 times as fast.  [4096, 2048] x [2048, 4096]
+// runs at 206-209 TFLOP/s of fp32 work = 1.24 PFLOP/s of bf16 (hipBLASLt's plain bf16 product
+// of that size: 1.09; the fp32 MFMA kernel that this replaced: 142 TFLOP/s).
 //
 // Special values.  An infinity, a NaN or a magnitude of 2^112 or more has a term x - h that
 // is not finite, and makes every output of its row or column NaN or infinite; so does a sum
