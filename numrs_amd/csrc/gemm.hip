@@ -832,9 +832,10 @@ bool shape_fits(const Gemm &g, bool xrc, bool yrc, int shape) {
   return ok;
 }
 
-double shape_us(const ShapeInfo &s, int64_t n, int64_t T) {
-  const int64_t left = n % s.most;
-  double t = (double)(n / s.most) * ((double)T * s.step[s.most] + s.fixed[s.most]);
+double shape_us(const ShapeInfo &s, int64_t n, int T) {
+  // most is 1, 2 or 3: no division by a variable
+  const int64_t full = s.most == 1 ? n : s.most == 2 ? n / 2 : n / 3, left = n - full * s.most;
+  double t = (double)full * ((double)T * s.step[s.most] + s.fixed[s.most]);
   if (left) t += (double)T * s.step[left] + s.fixed[left];
   return t;
 }
@@ -844,38 +845,58 @@ struct Plan {
   double t;
 };
 
-int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+template <typename T>
+T ceil_div(T a, T b) {
+  return (a + b - 1) / b;
+}
 
-int cut(int64_t k, int64_t T) {
-  const int64_t s = std::min<int64_t>(ceil_div(k, T), kMaxSplits);
-  return (int)ceil_div(k, ceil_div(k, s));
+// k tiles cut into ranges of at most T, of at most kMaxSplits: their number and length.
+struct Cut {
+  int n, len;
+};
+Cut cut(int k, int T) {
+  const int len = ceil_div(k, std::min(ceil_div(k, T), kMaxSplits));
+  return {ceil_div(k, len), len};
 }
 
 // Plan for a product a, or a pair with the TN product b in the same grid,
 // over `batch` batch entries, all cut alike.  Candidate tile lengths T are
 // ceil(k / s) for s = 1..kMaxSplits of either product; each product is cut
 // into ceil(k / T) ranges (none empty) and the smallest estimate wins, ties
-// going to the larger tile.
+// going to the larger tile.  This is host time of every call, so lengths that
+// repeat are passed over, and shapes whose steps alone, evenly over the CUs,
+// take longer than the best plan so far (a pair 10.2 -> 0.9-2.0 us, a product
+// 3.3 -> 0.5; the same plans).
 Plan plan_product(numrs_hip_ctx *ctx, const Gemm &a, bool xa, bool ya, const Gemm *b,
                   int64_t batch) {
   const int64_t cus = std::max(ctx->num_cus, 1);
   Plan best{-1, 1, 1, 0.0};
+  const int ka = ceil_div(a.R, kBR), kb = b ? ceil_div(b->R, kBR) : 0;
+  const double pa = 8.0 * batch * a.P * a.Q / kPartialBytesPerUs;  // a split's partials
+  const double pb = b ? 8.0 * batch * b->P * b->Q / kPartialBytesPerUs : 0.0;
   for (int shape = 0; shape < kShapeCount; ++shape) {
     if (!shape_fits(a, xa, ya, shape) || (b && !shape_fits(*b, false, false, shape))) continue;
     const ShapeInfo &s = kShapes[shape];
-    const int64_t ta = ceil_div(a.P, s.tp) * ceil_div(a.Q, s.tq), ka = ceil_div(a.R, kBR);
-    const int64_t tb = b ? ceil_div(b->P, s.tp) * ceil_div(b->Q, s.tq) : 0;
-    const int64_t kb = b ? ceil_div(b->R, kBR) : 0;
-    for (int cand = 0; cand < 2 * kMaxSplits; ++cand) {
-      if (cand >= kMaxSplits && !b) break;
-      const int64_t T = ceil_div(cand < kMaxSplits ? ka : kb, cand % kMaxSplits + 1);
-      const int sa = cut(ka, T), sb = b ? cut(kb, T) : 1;
-      const int64_t len = std::max(ceil_div(ka, sa), b ? ceil_div(kb, sb) : 0);
-      double t = shape_us(s, ceil_div((ta * sa + tb * sb) * batch, cus), len);
-      if (sa > 1) t += 8.0 * batch * sa * a.P * a.Q / kPartialBytesPerUs;
-      if (sb > 1) t += 8.0 * batch * sb * b->P * b->Q / kPartialBytesPerUs;
-      if (sa > 1 || sb > 1) t += kReduceUs;
-      if (best.shape < 0 || t < best.t) best = {shape, sa, sb, t};
+    const int64_t ta = (int64_t)ceil_div(a.P, s.tp) * ceil_div(a.Q, s.tq) * batch;
+    const int64_t tb = b ? (int64_t)ceil_div(b->P, s.tp) * ceil_div(b->Q, s.tq) * batch : 0;
+    double rate = s.step[1];  // of a tile and step, at best
+    for (int n = 2; n <= s.most; ++n) rate = std::min(rate, s.step[n] / n);
+    const double least = ((double)ta * ka + (double)tb * kb) / cus * rate;
+    if (best.shape >= 0 && least * 0.999 > best.t) continue;
+    for (int k : {ka, kb}) {
+      for (int c = 1, last = 0; c <= kMaxSplits && k > 0; ++c) {
+        const int T = ceil_div(k, c);
+        if (T == last) continue;
+        last = T;
+        const Cut ca = cut(ka, T), cb = b ? cut(kb, T) : Cut{1, 0};
+        const int64_t w = ta * ca.n + tb * cb.n;
+        const int64_t n = w <= 0x7fffffff ? (int64_t)ceil_div((uint32_t)w, (uint32_t)cus) : ceil_div(w, cus);
+        double t = shape_us(s, n, std::max(ca.len, cb.len));
+        if (ca.n > 1) t += ca.n * pa;
+        if (cb.n > 1) t += cb.n * pb;
+        if (ca.n > 1 || cb.n > 1) t += kReduceUs;
+        if (best.shape < 0 || t < best.t) best = {shape, ca.n, cb.n, t};
+      }
     }
   }
   return best;  // S fits every product
@@ -883,10 +904,10 @@ Plan plan_product(numrs_hip_ctx *ctx, const Gemm &a, bool xa, bool ya, const Gem
 
 // g as the plan's shape runs it.
 Gemm as_shape(Gemm g, int shape) {
-  g.tiles_p = (int)ceil_div(g.P, kShapes[shape].tp);
-  g.tiles_q = (int)ceil_div(g.Q, kShapes[shape].tq);
+  g.tiles_p = ceil_div(g.P, kShapes[shape].tp);
+  g.tiles_q = ceil_div(g.Q, kShapes[shape].tq);
   g.splits = 1;
-  g.ktiles_per_split = (int)ceil_div(g.R, kBR);
+  g.ktiles_per_split = ceil_div(g.R, kBR);
   g.partial = nullptr;
   return g;
 }
