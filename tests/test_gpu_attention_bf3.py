@@ -15,9 +15,8 @@ pytestmark = pytest.mark.gpu
 # (scores kept or formed again; four row groups: 512); heads of 8 (padded to 32), 24, 40 and 64, 72
 # (to 96) and 128; sequences one past, one short of and far from a block's end; 16 x 256 x 8 x 64 is
 # the encoder block's.  Both kinds of the backward's workgroups in one launch (without the output
-# after another for D): (2, 300, 16, 32), (2, 511, 8, 64) (on all CUs) and the small ones; a launch
-# each: (2, 300, 24, 32).  Below
-# 2^24 multiply-adds one launch of few workgroups: (1, 1, 1, 8) to (4, 128, 4, 64), and (2, 128, 1,
+# after another for D): (2, 300, 16, 32), (2, 511, 8, 64) and (1, 512, 16, 64) (on all CUs) and the
+# small ones; a launch each: (2, 300, 24, 32), (1, 513, 12, 64).  Below 2^24 multiply-adds one launch of few workgroups: (1, 1, 1, 8) to (4, 128, 4, 64), and (2, 128, 1,
 # 64), (1, 256, 7, 64), (1, 512, 2, 64; its backward takes the GEMMs); all of them GEMMs: (1, 192, 2,
 # 64), and heads of 96 on part of the chip.  (2, 200, 12, 32) and (8, 250, 20, 128): heads up to 32
 # on part of the chip and of 128 on all of it, with the scores kept.
@@ -25,7 +24,7 @@ SHAPES = [(4, 130, 8, 40), (16, 129, 16, 8), (2, 300, 16, 32), (8, 257, 12, 72),
           (3, 520, 30, 128), (10, 255, 10, 96), (5, 321, 7, 64), (16, 256, 8, 64), (4, 383, 24, 64),
           (2, 300, 16, 96), (2, 511, 8, 64), (2, 300, 24, 32), (1, 1, 1, 8), (3, 5, 2, 16), (2, 64, 3, 64),
           (1, 65, 2, 40), (1, 127, 5, 64), (4, 128, 4, 64), (2, 128, 1, 64), (1, 256, 7, 64), (1, 512, 2, 64),
-          (1, 384, 4, 56), (1, 192, 2, 64), (2, 200, 12, 32), (8, 250, 20, 128)]
+          (1, 512, 16, 64), (1, 513, 12, 64), (1, 384, 4, 56), (1, 192, 2, 64), (2, 200, 12, 32), (8, 250, 20, 128)]
 
 
 def _ref(q, k, v, g, B, S, H):
@@ -233,3 +232,33 @@ def test_backward_special_values(hip_ctx, B, S, H, dh, given):
     _same_kind(split(dv.numpy()), dV, "dv")
     _same_kind(split(dq.numpy()), dQ, "dq")
     _same_kind(split(dk.numpy()), dK, "dk")
+
+
+@pytest.mark.parametrize("B,S,H,dh", [(3, 5, 2, 16), (1, 127, 5, 64), (2, 128, 1, 40), (1, 256, 7, 64), (2, 300, 16, 32),
+                                      (8, 257, 12, 72)])
+def test_strides_and_addresses(hip_ctx, B, S, H, dh):
+    """Rows at odd strides, every buffer one float past a 16-byte boundary, forward and backward
+    with the output; what lies between the rows stays."""
+    print(f"[gpu] attention bf3 strides B={B} S={S} H={H} dh={dh}", flush=True)
+    rng = np.random.default_rng(S + dh)
+    D, c, lib = H * dh, hip_ctx, L.load()
+    li, lo, n = 3 * D + 5, D + 3, B * S
+    x, g, o0, d0 = rand(rng, (n, li)), rand(rng, (n, lo)), rand(rng, (n, lo)), rand(rng, (n, li))
+    q, k, v = x[:, :D], x[:, D:2 * D], x[:, 2 * D:3 * D]
+    P64, out64, *grads = _ref(q, k, v, g[:, :D], B, S, H)
+
+    def at(a):
+        return c.to_device(np.concatenate([np.zeros(1, np.float32), a.ravel()])).view(1, a.shape)
+
+    xd, gd, out, d = at(x), at(g), at(o0), at(d0)
+    P = at(np.full((B * H, S, S), np.nan, np.float32))
+    assert lib.numrs_hip_attention_forward_strided(c.handle, xd.ptr, _at(xd, D), _at(xd, 2 * D), li, P.ptr, out.ptr,
+                                                   lo, B, S, H, D) == 0
+    assert lib.numrs_hip_attention_backward_out_strided(
+        c.handle, xd.ptr, _at(xd, D), _at(xd, 2 * D), li, P.ptr, out.ptr, gd.ptr, lo, d.ptr, _at(d, D), _at(d, 2 * D),
+        B, S, H, D, 0) == 0
+    assert_contraction(P.numpy(), P64, dh, what="P")
+    got, gout = d.numpy(), out.numpy()
+    assert_contraction(gout[:, :D], out64, S, what="out")
+    assert_contraction(got[:, :3 * D], np.concatenate(grads, axis=1), S + dh, what="dq dk dv")
+    assert np.array_equal(gout[:, D:], o0[:, D:]) and np.array_equal(got[:, 3 * D:], d0[:, 3 * D:])
