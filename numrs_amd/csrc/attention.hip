@@ -9,9 +9,9 @@
 //   forward:   S = alpha * Q K^T,  P = softmax_rows(S),  O = P V
 //   backward:  dV = P^T dO,  dP = dO V^T,  dS = P * (dP - rowsum(dP*P)),
 //              dQ = alpha * dS K,  dK = alpha * dS^T Q
-// with alpha = 1/sqrt(dh).  The forward is one kernel and the backward two
-// (attention_bf3.h) where bf3_fits; other shapes take the batched GEMMs and the
-// one-wave-per-row softmax kernels.
+// with alpha = 1/sqrt(dh).  The forward is one kernel and the backward two, or
+// one (attention_bf3.h), where bf3_fits or bf3_few; other shapes take the batched
+// GEMMs and the one-wave-per-row softmax kernels.
 #include <algorithm>
 #include <cmath>
 

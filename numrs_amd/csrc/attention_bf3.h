@@ -427,11 +427,13 @@ struct RowStat {
     if (top == -INFINITY) return;  // no key of this lane yet
     l = l * __builtin_amdgcn_exp2f(m - top);
     m = top;
+    float part = 0.0f;  // a block's own sum: fewer roundings at l's size
 #pragma unroll
     for (int k = 0; k < N; ++k)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (WHOLE || key0 + 16 * k + e < S) l += __builtin_amdgcn_exp2f(sc.at<INF>(y[k][e], m));
+        if (WHOLE || key0 + 16 * k + e < S) part += __builtin_amdgcn_exp2f(sc.at<INF>(y[k][e], m));
+    l += part;
   }
   __device__ __forceinline__ static float part(float l, float m, float top) {
     return m == -INFINITY ? 0.0f : l * __builtin_amdgcn_exp2f(m - top);
